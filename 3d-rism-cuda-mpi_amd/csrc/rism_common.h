@@ -10,6 +10,23 @@
 
 namespace rism {
 
+// A pointer held in memory (a member of a kernel's by-value argument or of a
+// table), read as one to global memory.  The compiler only knows that of a
+// kernel's own pointer arguments; any other pointer, and a variable that may
+// hold either, it accesses with flat instructions, which also occupy the LDS
+// counter, so that each waits for every earlier load and LDS access (without
+// them: x pass of 160^3, 4 sites, 99 -> 88 us; y passes of 512^3, 4 sites,
+// 1.71 and 1.75 -> 1.56 and 1.67 ms).
+template <class T, class U>
+__device__ __forceinline__ T *global_ptr(U *const &p) {
+  return (T *)*reinterpret_cast<T __attribute__((address_space(1))) *const *>(&p);
+}
+
+// whether the flag of a solve that runs ahead of the host is up (Params::done)
+__device__ __forceinline__ bool stopped(const int *const &done) {
+  return done && *global_ptr<const int>(done);
+}
+
 __device__ __forceinline__ double rexp(double a) { return exp(a); }
 __device__ __forceinline__ float rexp(float a) { return expf(a); }
 

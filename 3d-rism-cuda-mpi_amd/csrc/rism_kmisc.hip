@@ -18,9 +18,9 @@ __global__ void __launch_bounds__(256)
   __shared__ double sh[256];
   if (grp) {  // grouped launch: this context's partial sums
     const GroupPtrs &g = grp[blockIdx.z];
-    done = g.done;
-    in = g.partial;
-    out = g.sums;
+    done = global_ptr<const int>(g.done);
+    in = global_ptr<const double>(g.partial);
+    out = global_ptr<double>(g.sums);
   }
   if (done && *done) return;
   const int col = blockIdx.x;
@@ -101,11 +101,11 @@ __global__ void k_an2_picard(V16<Re> *__restrict__ tnew, const V16<Re> *__restri
                              size_t nv, const int *done, const GroupPtrs *grp) {
   if (grp) {
     const GroupPtrs &g = grp[blockIdx.z];
-    done = g.done;
-    tnew = (V16<Re> *)g.tnew;
-    t = (const V16<Re> *)g.t;
-    R = (const V16<Re> *)g.R;
-    Pb = (V16<Re> *)g.Pb;
+    done = global_ptr<const int>(g.done);
+    tnew = global_ptr<V16<Re>>(g.tnew);
+    t = global_ptr<const V16<Re>>(g.t);
+    R = global_ptr<const V16<Re>>(g.R);
+    Pb = global_ptr<V16<Re>>(g.Pb);
   }
   if (done && *done) return;
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -130,14 +130,14 @@ __global__ void k_an2_update(V16<Re> *__restrict__ tnew, const V16<Re> *__restri
                              Re mcoef, size_t nv, const int *done, const GroupPtrs *grp) {
   if (grp) {
     const GroupPtrs &g = grp[blockIdx.z];
-    done = g.done;
-    tnew = (V16<Re> *)g.tnew;
-    t = (const V16<Re> *)g.t;
-    R = (const V16<Re> *)g.R;
-    P0 = (const V16<Re> *)g.P0;
-    P1 = (const V16<Re> *)g.P1;
-    Pb = (V16<Re> *)g.Pb;
-    scal = g.scal;
+    done = global_ptr<const int>(g.done);
+    tnew = global_ptr<V16<Re>>(g.tnew);
+    t = global_ptr<const V16<Re>>(g.t);
+    R = global_ptr<const V16<Re>>(g.R);
+    P0 = global_ptr<const V16<Re>>(g.P0);
+    P1 = global_ptr<const V16<Re>>(g.P1);
+    Pb = global_ptr<V16<Re>>(g.Pb);
+    scal = global_ptr<const double>(g.scal);
   }
   if (done && *done) return;
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -166,10 +166,10 @@ __global__ void k_step_finish(const double *__restrict__ sums, const double *__r
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
   if (grp) {
     const GroupPtrs &g = grp[blockIdx.z];
-    sums = g.sums;
-    scal = g.scal;
-    rms_hist = g.rms_hist;
-    done = g.done;
+    sums = global_ptr<const double>(g.sums);
+    scal = global_ptr<double>(g.scal);
+    rms_hist = global_ptr<double>(g.rms_hist);
+    done = global_ptr<int>(g.done);
   }
   if (done && done[0]) return;
   // step number: done[2] counts the finished steps of the run
@@ -355,7 +355,7 @@ __global__ void k_andm_update(V16<Re> *__restrict__ tnew, const V16<Re> *__restr
   for (int h = 0; h < RISM_MAX_HIST; ++h) {
     if (h < H.nh) {
       // Pb may be the oldest P_h: this thread reads element i before it writes it
-      const V16<Re> p = ld_nt(reinterpret_cast<const V16<Re> *>(H.p[h]) + i);
+      const V16<Re> p = ld_nt(global_ptr<const V16<Re>>(H.p[h]) + i);
       const Re x = (Re)xcoef[h];
 #pragma unroll
       for (int k = 0; k < V16<Re>::K; ++k) a.a[k] = fma(x, p.a[k] - q.a[k], a.a[k]);

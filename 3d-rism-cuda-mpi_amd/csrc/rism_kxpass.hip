@@ -174,11 +174,11 @@ __global__ void __launch_bounds__(512)
   constexpr int T = FftShape<L>::T, CS = FftShape<L>::CS;
   C *lds = reinterpret_cast<C *>(xsm);
   if (P.grp) {  // grouped launch: this context's spectrum and fk
-    const GroupPtrs &g = P.grp[blockIdx.z];
-    if (g.done && *g.done) return;
-    spec = (C *)g.spec;
-    fkraw = (const C *)g.fk;
-  } else if (P.done && *P.done) return;
+    const GroupPtrs &g = global_ptr<const GroupPtrs>(P.grp)[blockIdx.z];
+    if (stopped(g.done)) return;
+    spec = global_ptr<C>(g.spec);
+    fkraw = global_ptr<const C>(g.fk);
+  } else if (stopped(P.done)) return;
   const int tid = threadIdx.x;
   const int nv = P.natv;
   // row slots: a workgroup of short rows (T < 64) holds several row pairs

@@ -17,8 +17,8 @@ __global__ void __launch_bounds__(B *FftShape<L>::T)
   __shared__ C lds[B * CS];
   if (grp) {  // grouped launch: this context's spectrum
     const GroupPtrs &g = grp[blockIdx.z];
-    done = g.done;
-    spec = (C *)g.spec;
+    done = global_ptr<const int>(g.done);
+    spec = global_ptr<C>(g.spec);
   }
   if (done && *done) return;
   const int tid = threadIdx.x;

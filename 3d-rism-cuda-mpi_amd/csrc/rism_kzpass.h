@@ -49,13 +49,13 @@ __global__ void __launch_bounds__(B *TZ)
   constexpr int T = TZ, CS = FftShape<M>::CS;
   __shared__ C lds[B * CS];
   if (P.grp) {  // grouped launch: this context's fields
-    const GroupPtrs &g = P.grp[blockIdx.z];
-    if (g.done && *g.done) return;
-    t = (const Re *)g.t;
-    u = (const Re *)g.u;
-    fr = (const Re *)g.fr;
-    spec = (C *)g.spec;
-  } else if (P.done && *P.done) return;
+    const GroupPtrs &g = global_ptr<const GroupPtrs>(P.grp)[blockIdx.z];
+    if (stopped(g.done)) return;
+    t = global_ptr<const Re>(g.t);
+    u = global_ptr<const Re>(g.u);
+    fr = global_ptr<const Re>(g.fr);
+    spec = global_ptr<C>(g.spec);
+  } else if (stopped(P.done)) return;
   const int tid = threadIdx.x;
   const int c = tid % B, j = tid / B;
   // logical workgroup order: site fastest, then x tile, then y (sites of
@@ -250,16 +250,16 @@ __global__ void __launch_bounds__(B *TZ)
   constexpr int LDSN = (B * CS > NC) ? B * CS : NC;
   __shared__ C lds[LDSN];
   if (P.grp) {  // grouped launch (AN2 and Picard steps): this context's fields
-    const GroupPtrs &g = P.grp[blockIdx.z];
-    if (g.done && *g.done) return;
-    spec = (const C *)g.spec;
-    t = (const Re *)g.t;
-    u = (const Re *)g.u;
-    R = (Re *)g.R;
-    R0 = (const Re *)g.R0;
-    R1 = (const Re *)g.R1;
-    partial = g.partial;
-  } else if (P.done && *P.done) return;
+    const GroupPtrs &g = global_ptr<const GroupPtrs>(P.grp)[blockIdx.z];
+    if (stopped(g.done)) return;
+    spec = global_ptr<const C>(g.spec);
+    t = global_ptr<const Re>(g.t);
+    u = global_ptr<const Re>(g.u);
+    R = global_ptr<Re>(g.R);
+    R0 = global_ptr<const Re>(g.R0);
+    R1 = global_ptr<const Re>(g.R1);
+    partial = global_ptr<double>(g.partial);
+  } else if (stopped(P.done)) return;
   const int tid = threadIdx.x;
   const int c = tid % B, j = tid / B;
   const int ntx = (P.nx + B - 1) / B;
@@ -364,8 +364,8 @@ __global__ void __launch_bounds__(B *TZ)
       for (int q = 0; q < RISM_MAX_HIST; ++q)
         if (q < H.nh) {
           // non-temporal in FP64 (-3 %); in the spilling FP32 tile it measured slower
-          const Re hq = (sizeof(Re) == 8) ? __builtin_nontemporal_load(&H.r[q][voff + i])
-                                          : H.r[q][voff + i];
+          const Re *hp = global_ptr<const Re>(H.r[q]) + (voff + i);
+          const Re hq = (sizeof(Re) == 8) ? __builtin_nontemporal_load(hp) : *hp;
           s[1 + q] += r * (double)hq;
         }
     }
