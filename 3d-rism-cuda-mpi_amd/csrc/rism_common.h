@@ -134,6 +134,15 @@ struct ZTile {
   static constexpr int BF = R4F ? 1024 / TF : B;
 };
 
+// x when A, else y (two objects of different types)
+template <bool A, class X, class Y>
+__device__ __forceinline__ auto &pick_ref(X &x, Y &y) {
+  if constexpr (A)
+    return x;
+  else
+    return y;
+}
+
 static inline unsigned nblk(size_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
 // Workgroups of a 1D grid are handed to the 8 XCDs of the MI355X round-robin

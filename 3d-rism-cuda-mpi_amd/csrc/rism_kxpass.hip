@@ -150,6 +150,25 @@ __device__ __forceinline__ void oz_points_reg(cx<Re> *lds, int CS, const int (&o
   }
 }
 
+// the first stage's elements of one row, pre-twiddled (zeros for a spare row)
+template <class Re>
+struct RowLoad {
+  using staged = void;
+  using raw_t = cx<Re>;
+  enum { group = 8 };
+  const cx<Re> *row, *px;
+  cx<Re> prej;
+  int j;
+  bool spare;
+  __device__ __forceinline__ cx<Re> fetch(int i) const {
+    return cx<Re>{__builtin_nontemporal_load(&row[i].x), __builtin_nontemporal_load(&row[i].y)};
+  }
+  __device__ __forceinline__ cx<Re> make(cx<Re> a, int i) const {
+    const cx<Re> w = cmul(a, cmul(prej, px[i - j]));
+    return spare ? cx<Re>{0, 0} : w;
+  }
+};
+
 // One workgroup per m and pair of mirror rows (y, ny-1-y) -- several pairs
 // side by side for short rows, see the row slots below -- all sites: natv
 // columns of nx complex in LDS per pair, natv * T threads per pair, the two
@@ -239,12 +258,8 @@ __global__ void __launch_bounds__(512)
         if (!kSlots && !rowok) break;
         const size_t rowoff = rowok ? ((size_t)m * P.ny + (r ? y1 : y0)) * L : 0;
         C *row = spec + (size_t)v * rowstride + rowoff;
-        auto load = [&](int i) -> C {
-          // rowoff is 0 for a spare row: the load stays in bounds, unguarded
-          const C a{__builtin_nontemporal_load(&row[i].x), __builtin_nontemporal_load(&row[i].y)};
-          const C w = cmul(a, cmul(prej, px[i - j]));
-          return (kSlots && !rowok) ? C{0, 0} : w;
-        };
+        // rowoff is 0 for a spare row: the loads stay in bounds, unguarded
+        RowLoad<Re> load{row, px, prej, j, kSlots && !rowok};
         auto store = [&](int i, C vv) {
           if (kSlots && !rowok) return;
           const C o = cmulc(vv, cmul(prej, px[i - j]));
@@ -285,12 +300,8 @@ __global__ void __launch_bounds__(512)
     const int y = r ? y1 : y0;
     const size_t rowoff = rowok ? ((size_t)m * P.ny + y) * L : 0;
     C *row = spec + (size_t)v * rowstride + rowoff;
-    auto load = [&](int i) -> C {
-      // rowoff is 0 for a spare row: the load stays in bounds, unguarded
-      const C a{__builtin_nontemporal_load(&row[i].x), __builtin_nontemporal_load(&row[i].y)};
-      const C w = cmul(a, cmul(prej, px[i - j]));
-      return (kSlots && !rowok) ? C{0, 0} : w;
-    };
+    // rowoff is 0 for a spare row: the loads stay in bounds, unguarded
+    RowLoad<Re> load{row, px, prej, j, kSlots && !rowok};
     auto store = [&](int i, C vv) {
       if (kSlots && !rowok) return;
       const C o = cmulc(vv, cmul(prej, px[i - j]));

@@ -34,12 +34,31 @@ __global__ void __launch_bounds__(B *FftShape<L>::T)
   // col points at column 0 when x is past nx, so every load stays in bounds
   // and is issued unguarded: a load guarded by `ok` waits for its data inside
   // the guard, one element after another
-  auto load = [&](int i) -> C {
-    const C *q = col + (size_t)i * nx;
-    const C vv{__builtin_nontemporal_load(&q->x), __builtin_nontemporal_load(&q->y)};
-    const C w = (S < 0) ? cmul(vv, cmul(prej, pre[i - j])) : vv;
-    return ok ? w : C{0, 0};
+  struct Rows {
+    using staged = void;
+    using raw_t = C;
+    enum { group = 8 };
+    const C *col;
+    const C *pre;
+    C prej;
+    int nx, j;
+    bool ok;
+    __device__ __forceinline__ C fetch(int i) const {
+      const C *q = col + (size_t)i * nx;
+      return C{__builtin_nontemporal_load(&q->x), __builtin_nontemporal_load(&q->y)};
+    }
+    __device__ __forceinline__ C make(C vv, int i) const {
+      const C w = cmul(vv, cmul(prej, pre[i - j]));
+      return ok ? w : C{0, 0};
+    }
+  } fwd{col, pre, prej, nx, j, ok};
+  // the inverse has nothing to form from its elements, and its loads are
+  // issued together without the staging
+  auto inv = [&](int i) -> C {
+    const C vv = fwd.fetch(i);
+    return ok ? vv : C{0, 0};
   };
+  auto &load = pick_ref<(S < 0)>(fwd, inv);
   auto store = [&](int i, C vv) {
     if (!ok) return;
     const C o = (S < 0) ? vv : cmulc(vv, cmul(prej, pre[i - j]));

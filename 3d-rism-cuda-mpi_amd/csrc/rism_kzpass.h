@@ -28,15 +28,6 @@ enum ZKind {
   ZK_PLAIN = 3,   // plain transform of t (forward) or to h (inverse)
 };
 
-// x when A, else y (two objects of different types)
-template <bool A, class X, class Y>
-__device__ __forceinline__ auto &pick_ref(X &x, Y &y) {
-  if constexpr (A)
-    return x;
-  else
-    return y;
-}
-
 // WPE: waves per SIMD the kernel is compiled for (register budget)
 template <int M, int B, int TZ, int MAXR, int KIND, class Re, int WPE = (MAXR == 4 ? 8 : 1)>
 __global__ void __launch_bounds__(B *TZ)
@@ -186,10 +177,10 @@ __global__ void __launch_bounds__(B *TZ)
         }
       }
     } store{out, mstride, zpre, zpost[j], zpost[NS - 1 - j], ok};
-    fft_column<M, -1, true, true, TZ, MAXR>(col, j, twM, load, store);
+    fft_column<M, -1, true, true, TZ, MAXR, (WPE <= 2)>(col, j, twM, load, store);
   } else {
     auto store = [&](int, C) {};
-    fft_column<M, -1, true, false, TZ, MAXR>(col, j, twM, load, store);
+    fft_column<M, -1, true, false, TZ, MAXR, (WPE <= 2)>(col, j, twM, load, store);
     // zpost[m] = e^{-i pi (2m+1)/nz} = zpost[j] zpre[m - j]
     const C zpostj = zpost[j];
     for (int m = j; m < M; m += T) {
@@ -449,7 +440,7 @@ __global__ void __launch_bounds__(B *TZ)
       }
     } store{tv,   uv,   R0v,  R1v,   r0 ? r0 + voff : nullptr, Rv, zpre, zpre[j], j, base,
             plane, scale, clos, ok, {}};
-    fft_column<M, +1, false, true, TZ, MAXRI>(col, j, twM, load, store);
+    fft_column<M, +1, false, true, TZ, MAXRI, (WPE <= 2)>(col, j, twM, load, store);
 #pragma unroll
     for (int k = 0; k < W; ++k) s[k] = store.s[k];
   } else {
@@ -460,7 +451,7 @@ __global__ void __launch_bounds__(B *TZ)
       resid(2 * p, zz.x);
       resid(2 * p + 1, zz.y);
     };
-    fft_column<M, +1, false, true, TZ, MAXRI>(col, j, twM, load, store);
+    fft_column<M, +1, false, true, TZ, MAXRI, (WPE <= 2)>(col, j, twM, load, store);
   }
 
   // workgroup reduction of the W sums: wave shuffles then LDS when the
