@@ -367,10 +367,14 @@ int make_chi(rism_ctx *c, const rism_solvent *s) {
   c->P.np = np;
   c->P.x0 = xk[0];
   c->P.idk = 1.0 / dk;
-  // cubic box: every |k|^2 is (pi/L)^2 (ox^2 + oy^2 + oz^2) with odd o, i.e.
-  // (pi/L)^2 (8 i + 3); tabulate chi once per shell i
-  c->P.shell = 0;
-  if (!c->opts.chi_spline && c->box[0] == c->box[1] && c->box[1] == c->box[2]) {
+  // chi is tabulated once per context unless the caller asks for the spline.
+  // Cubic box: every |k|^2 is (pi/L)^2 (ox^2 + oy^2 + oz^2) with odd o, i.e.
+  // (pi/L)^2 (8 i + 3): one row per shell i.
+  // Other boxes: one row per point of an octant (without memory for it, the
+  // spline).
+  c->P.shell = RISM_CHI_SPLINE;
+  if (c->opts.chi_spline) return RISM_OK;
+  if (c->box[0] == c->box[1] && c->box[1] == c->box[2]) {
     const long smax = (long)(c->nx - 1) * (c->nx - 1) + (long)(c->ny - 1) * (c->ny - 1) +
                       (long)(c->nz - 1) * (c->nz - 1);
     const size_t nshell = (size_t)((smax - 3) / 8 + 1);
@@ -378,8 +382,26 @@ int make_chi(rism_ctx *c, const rism_solvent *s) {
     c->nchitab = nshell * nv2;
     HIPCHECK(rism::run_chi_table(c->knots, c->coef, c->P, M_PI / c->box[0], nshell, c->chitab, c->st));
     HIPCHECK(hipStreamSynchronize(c->st));
-    c->P.shell = 1;
+    c->P.shell = RISM_CHI_SHELL;
   }
+  return RISM_OK;
+}
+
+// The octant table of a box with different sides, for both levels.  It is
+// allocated after everything that the context needs; without memory for it
+// the x pass evaluates the spline.
+int make_chi_octant(rism_ctx *c) {
+  if (c->opts.chi_spline || c->P.shell != RISM_CHI_SPLINE) return RISM_OK;
+  const size_t n = (size_t)(c->nx / 2) * (c->ny / 2) * (c->nz / 2) * c->natv * c->natv;
+  double *tab = nullptr;
+  float *tab32 = nullptr;
+  if (c->alloc(&tab, n) || (c->opts.precision == 1 && c->alloc(&tab32, n))) return RISM_OK;
+  HIPCHECK(rism::run_chi_octant(c->knots, c->coef, c->P, tab, c->st));
+  if (tab32) HIPCHECK(rism::run_convert((const double *)tab, tab32, n, c->st));
+  c->d.chitab = c->chitab = tab;
+  c->f.chitab = tab32;
+  c->nchitab = n;
+  c->P.shell = RISM_CHI_OCTANT;
   return RISM_OK;
 }
 
@@ -1697,6 +1719,7 @@ rism_ctx *rism_create(const rism_grid *grid, const rism_solvent *solvent,
   if (hipHostMalloc((void **)&c->hscal, 8 * sizeof(double)) != hipSuccess ||
       hipHostMalloc((void **)&c->hflag, 3 * sizeof(int)) != hipSuccess)
     return fail(rism::set_error(RISM_ERR_NOMEM, "hipHostMalloc failed"));
+  if ((rc = make_chi_octant(c))) return fail(rc);
   if (tune::enabled() || tune::forced(0) >= 0) {
     if ((rc = tune_level<double>(c))) return fail(rc);
     if (c->opts.precision == 1 && (rc = tune_level<float>(c))) return fail(rc);

@@ -5,6 +5,12 @@
 
 #define RISM_MAX_SITES 16
 
+// chi_vv(|k|) of the OZ step: the spline evaluated at |k|, the table of the
+// k^2 shells of a cubic box, or the table of the points kx, ky, kz > 0
+#define RISM_CHI_SPLINE 0
+#define RISM_CHI_SHELL 1
+#define RISM_CHI_OCTANT 2
+
 namespace rism {
 
 template <class Re>
@@ -39,7 +45,7 @@ struct Params {
   int clos;          // 0 KH, 1 HNC
   int mode;          // 0 solver step; 1 plain forward transform; 2 plain inverse;
                      // 3 difference-form step (correction sweep of the mixed solve)
-  int shell;         // 1: chi from the cubic-box shell table, 0: spline at |k|
+  int shell;         // chi source: RISM_CHI_SPLINE, _SHELL or _OCTANT
   double dv;         // volume element (forward scale)
   double inv_scale;  // 1 / (dv nx ny (nz/2)): inverse scale of the three passes
   double dr[3];      // grid spacing
@@ -100,13 +106,16 @@ hipError_t run_zfwd(const Params &P, const Re *t, const Re *u, const Re *fr, cx<
 template <class Re>
 hipError_t run_y(const Params &P, cx<Re> *spec, int dir, const cx<Re> *twL, const cx<Re> *pre,
                  hipStream_t st);
-// chitab: the cubic-box shell table in the bulk type (P.shell = 1)
+// chitab: the shell or octant table in the bulk type (P.shell != 0)
 template <class Re>
 hipError_t run_xoz(const Params &P, cx<Re> *spec, const cx<Re> *fkraw, const cx<Re> *twL,
                    const cx<Re> *prex, const double *knots, const double *coef,
                    const Re *chitab, hipStream_t st);
 hipError_t run_chi_table(const double *knots, const double *coef, const Params &P,
                          double kscale, size_t nshell, double *out, hipStream_t st);
+// out: natv^2 (nx/2) (ny/2) (nz/2) values, [m][yh][pair][xh]
+hipError_t run_chi_octant(const double *knots, const double *coef, const Params &P, double *out,
+                          hipStream_t st);
 // AN2 partial sums (6 per workgroup) of the residual pass
 // P.mode 3 (difference form): t = correction d, u = exponent a = -u + t0 at
 // the base point, r0 = the full residual at t0; R = r0 + h - (g(a+d) - g(a)).

@@ -34,16 +34,38 @@ namespace rism {
 // ---------------------------------------------------------------------------
 // 3. DFT along x, OZ with chi_vv(|k|), inverse DFT along x
 // ---------------------------------------------------------------------------
-// chi_vv(|k|) sources for the OZ step.  ChiTable: the cubic-box shell table
-// (one row of natv^2 values per k^2 shell, built once by k_chi_table);
-// ChiSpline: the natural cubic spline of the .xvk table evaluated at |k|
+// chi_vv(|k|) sources for the OZ step.  ChiTable: a table built once per
+// context, one row of natv^2 values per k^2 shell for a cubic box
+// (k_chi_table), or one per point of the octant kx, ky, kz > 0 for a box with
+// different sides (k_chi_octant; |k| has few repeats there).  ChiSpline: the
+// natural cubic spline of the .xvk table evaluated at |k|
 // (solvent_spline.cu:44-55 evaluates the same spline at the same |k| shell
 // values; splint.cc:4-20 picks the interval).
-template <class Tb>
+// The octant table holds natv^2 / 8 words per grid point, which the pass
+// reads once a step, and against it stood four coefficient gathers, a square
+// root and a knot search per k and pair of sites: 144 x 160 x 128, 4 sites,
+// 124 -> 79 us; 72 x 90 x 60, 2 sites, 17 -> 9 us.
+template <class Tb, int STRIDE>
 struct ChiTable {
   const Tb *row;
-  __device__ __forceinline__ Tb operator()(int pw) const { return row[pw]; }
+  __device__ __forceinline__ Tb operator()(int pw) const { return row[pw * STRIDE]; }
 };
+// the table's row for the points (+-kx, +-ky) at x index jx < L/2, y index
+// yh < ny/2 and plane m.  Shells are rows of consecutive values; in the
+// octant the x index is fastest, so that neighbouring threads read
+// neighbouring words.
+template <int L, int CHI, class Tb>
+__device__ __forceinline__ auto chi_row(const Tb *tab, const Params &P, int nv2, int jx, int yh,
+                                        int m) {
+  if constexpr (CHI == RISM_CHI_OCTANT) {
+    return ChiTable<Tb, L / 2>{tab + ((size_t)m * (P.ny / 2) + yh) * nv2 * (L / 2) + jx};
+  } else {
+    // |k|^2 = (pi/L)^2 (8 sidx + 3)
+    const long ox = 2 * jx - L + 1, oy = 2 * yh - P.ny + 1, oz = 2 * m + 1;
+    const long sidx = (ox * ox + oy * oy + oz * oz - 3) >> 3;
+    return ChiTable<Tb, 1>{tab + sidx * nv2};
+  }
+}
 struct ChiSpline {
   const double *cf;
   double tt;
@@ -91,9 +113,9 @@ __device__ __forceinline__ void oz_points(cx<Re> *lds, int CS, const int (&off)[
   }
 }
 
-// NVMAX (4 or 8) bounds the site counts compiled into one kernel: the
-// register allocation follows the largest case, so natv <= 4 gets a kernel
-// without the 5..8-site paths.
+// NVMAX (2, 4 or 8) bounds the site counts compiled into one kernel: the
+// register allocation follows the largest case, so few sites get a kernel
+// without the paths of more.
 template <int NVMAX, int NP, class Re, class Chi>
 __device__ __forceinline__ void oz_dispatch(cx<Re> *lds, int CS, const int (&off)[NP],
                                             const cx<Re> (&fk)[NP], const Params &P,
@@ -101,8 +123,12 @@ __device__ __forceinline__ void oz_dispatch(cx<Re> *lds, int CS, const int (&off
   switch (P.natv) {
     case 1: oz_points<1>(lds, CS, off, fk, P, 1, X); break;
     case 2: oz_points<2>(lds, CS, off, fk, P, 2, X); break;
-    case 3: oz_points<3>(lds, CS, off, fk, P, 3, X); break;
-    case 4: oz_points<4>(lds, CS, off, fk, P, 4, X); break;
+    case 3:
+      if constexpr (NVMAX > 2) oz_points<3>(lds, CS, off, fk, P, 3, X);
+      break;
+    case 4:
+      if constexpr (NVMAX > 2) oz_points<4>(lds, CS, off, fk, P, 4, X);
+      break;
     default:
       if constexpr (NVMAX > 4) {
         switch (P.natv) {
@@ -126,12 +152,13 @@ __device__ __forceinline__ void oz_row(cx<Re> *lds, int CS, int jx, int L, const
 }
 
 // The same contraction with the chi row already in registers (chr[v][w],
-// v, w < NV): used when every thread owns at most one (kx, -kx) pair, so the
-// row is fetched before the forward transform and its latency is hidden.
-template <int NV, class Re>
+// v, w < NV): used when every thread owns at most kChiPairs (kx, -kx) pairs,
+// so the rows are fetched before the forward transform and their latency is
+// hidden.
+template <int NV, int NVM, class Re>
 __device__ __forceinline__ void oz_points_reg(cx<Re> *lds, int CS, const int (&off)[2],
                                               const cx<Re> (&fk)[2], const Params &P,
-                                              const Re (&chr)[4][4]) {
+                                              const Re (&chr)[NVM][NVM]) {
   cx<Re> c[2][NV];
 #pragma unroll
   for (int w = 0; w < NV; ++w) {
@@ -174,21 +201,43 @@ struct RowLoad {
 // columns of nx complex in LDS per pair, natv * T threads per pair, the two
 // rows one after the other.  The rows of a pair have the same |ky| and so the same chi rows
 // (the shell index and |k| depend on ky^2 only): the register path loads
-// them once for both rows.  SHELL selects the chi source at compile time (the
-// cubic-box shell table or the spline at |k|) and NVMAX bounds the site
-// count, so each instantiation carries only the registers it needs.
+// them once for both rows.  CHI selects the chi source at compile time (the
+// shell or octant table or the spline at |k|) and NVMAX bounds the site
+// count, so each instantiation carries only the registers it needs (both
+// tables in one kernel: 160 points 168 -> 176 VGPRs, two waves per SIMD
+// instead of three, 88 -> 156 us at 160^3).
 // dynamic LDS of the x passes, shared by all instantiations; 16-byte
 // aligned, so FP64 complex values move as ds_read_b128 / ds_write_b128
 // (with the default 8-byte alignment they split into ds_read2_b64 pairs,
 // with about eight bank-conflict cycles per LDS instruction)
 extern __shared__ __attribute__((aligned(16))) double xsm[];
 
-template <int L, int NVMAX, bool SHELL, class Re>
+// (kx, -kx) pairs per thread whose chi rows are kept in registers: one row of
+// 16 values for 3 and 4 sites, two of 4 for up to 2 sites, whose rows have
+// half as many threads
+template <int NVMAX>
+constexpr int kChiPairs = NVMAX == 2 ? 2 : 1;
+
+// waves of a launch from which rows are taken in pairs: below, the rows of a
+// pair run side by side in workgroups of their own (64^3, 2 sites, 256 waves
+// in pairs: 9.8 -> 6.5 us, with the 2-site kernel)
+constexpr long kPairedWaves = 2048;
+
+// The FP64 table kernels of up to 4 sites are held to 168 VGPRs, three waves
+// per SIMD (160 points took 170: 86 -> 102 us at 160^3); rows of 36 and 72
+// points would spill 17 for it (8.8 -> 10.3 us at 72 x 90 x 60) and are not.
+template <int L, int NVMAX, int CHI, class Re>
+constexpr int xoz_waves_per_eu() {
+  return (sizeof(Re) == 8 && CHI != RISM_CHI_SPLINE && NVMAX <= 4 && L >= 80) ? 3 : 1;
+}
+
+template <int L, int NVMAX, int CHI, class Re>
 __global__ void __launch_bounds__(512)
+    __attribute__((amdgpu_waves_per_eu(xoz_waves_per_eu<L, NVMAX, CHI, Re>())))
     k_xpass_oz(cx<Re> *__restrict__ spec, const cx<Re> *__restrict__ fkraw, Params P,
                const cx<Re> *__restrict__ twL, const cx<Re> *__restrict__ prex,
                const double *__restrict__ knots, const double *__restrict__ coef,
-               const Re *__restrict__ chitab) {
+               const Re *__restrict__ chitab, int paired) {
   using C = cx<Re>;
   constexpr int T = FftShape<L>::T, CS = FftShape<L>::CS;
   C *lds = reinterpret_cast<C *>(xsm);
@@ -210,9 +259,11 @@ __global__ void __launch_bounds__(512)
   const int v = tl / T, j = tl % T;
   const int y0 = kSlots ? blockIdx.x * (int)(blockDim.x / nthr) + slot : (int)blockIdx.x;
   const int m = blockIdx.y;
-  const bool live = !kSlots || y0 < (P.ny + 1) / 2;  // the last workgroup's slots may be spare
-  const int y1 = P.ny - 1 - y0;                       // the mirror row
-  const bool pair = live && y1 > y0;                  // not for the middle row of odd ny
+  // the last workgroup's slots may be spare
+  const bool live = !kSlots || y0 < (paired ? (P.ny + 1) / 2 : P.ny);
+  const int y1 = P.ny - 1 - y0;                  // the mirror row
+  const bool pair = paired && live && y1 > y0;   // not for the middle row of odd ny
+  const int yh = y0 < y1 ? y0 : y1;              // chi row of both
   const int M = P.nz / 2;
   const size_t rowstride = (size_t)M * P.ny * L;  // site stride in spec
   C *slds = lds + slot * nv * CS;
@@ -225,25 +276,29 @@ __global__ void __launch_bounds__(512)
   const C prej = prex[j];
   auto nostore = [&](int, C) {};
   const int nv2 = nv * nv;
-  const long oy = 2 * y0 - P.ny + 1, oz = 2 * m + 1;  // odd lattice coordinates (|oy| of both rows)
   // With several slots both rows are run by every slot (a spare row
   // transforms zeros and stores nothing), so that all threads meet the same
   // barriers.
-  // at most one (kx, -kx) pair per thread and at most 4 sites: fetch this
-  // thread's chi row (shared by the two rows) and the fk pair of each row
-  // before its forward transform
-  if constexpr (SHELL && NVMAX == 4) {
-    if (L / 2 <= nthr) {
-      Re chr[4][4];
-      const bool mine = live && tl < L / 2;
-      if (mine) {
-        const long ox = 2 * tl - L + 1;
-        const long sidx = (ox * ox + oy * oy + oz * oz - 3) >> 3;
-        const Re *rowp = chitab + sidx * nv2;
+  // few (kx, -kx) pairs per thread and at most 4 sites: fetch this thread's
+  // chi rows (shared by the two rows) and the fk pairs of each row before its
+  // forward transform
+  if constexpr (CHI != RISM_CHI_SPLINE && NVMAX <= 4) {
+    constexpr int NP = kChiPairs<NVMAX>;
+    if (L / 2 <= NP * nthr) {
+      Re chr[NP][NVMAX][NVMAX];
+      bool mine[NP];
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
+      for (int k = 0; k < NP; ++k) {
+        const int jx = tl + k * nthr;
+        mine[k] = live && jx < L / 2;
+        if (mine[k]) {
+          const auto X = chi_row<L, CHI>(chitab, P, nv2, jx, yh, m);
 #pragma unroll
-          for (int w = 0; w < 4; ++w) chr[v][w] = (v < nv && w < nv) ? rowp[v * nv + w] : (Re)0;
+          for (int v = 0; v < NVMAX; ++v)
+#pragma unroll
+            for (int w = 0; w < NVMAX; ++w)
+              chr[k][v][w] = (v < nv && w < nv) ? X(v * nv + w) : (Re)0;
+        }
       }
 #pragma unroll 1
       for (int r = 0; r < 2; ++r) {
@@ -255,7 +310,7 @@ __global__ void __launch_bounds__(512)
         // a spare row: the workgroup stops before it (one slot), or the slot
         // runs it on zeros (several slots: per-element guards)
         const bool rowok = r ? pair : live;
-        if (!kSlots && !rowok) break;
+        if ((!kSlots && !rowok) || (r && !paired)) break;
         const size_t rowoff = rowok ? ((size_t)m * P.ny + (r ? y1 : y0)) * L : 0;
         C *row = spec + (size_t)v * rowstride + rowoff;
         // rowoff is 0 for a spare row: the loads stay in bounds, unguarded
@@ -268,20 +323,31 @@ __global__ void __launch_bounds__(512)
         };
         // the difference-form step (mode 3): the long-range term cancels, fk = 0
         const C *fkr = (P.mode == 3) ? nullptr : fkraw + rowoff;
-        C fkp[2] = {C{0, 0}, C{0, 0}};
-        if (mine && rowok && fkr) {
-          fkp[0] = fkr[tl];
-          fkp[1] = fkr[L - 1 - tl];
+        C fkp[NP][2];
+#pragma unroll
+        for (int k = 0; k < NP; ++k) {
+          const int jx = tl + k * nthr;
+          const bool rd = mine[k] && rowok && fkr;
+          fkp[k][0] = rd ? fkr[jx] : C{0, 0};
+          fkp[k][1] = rd ? fkr[L - 1 - jx] : C{0, 0};
         }
         if (r) __syncthreads();  // the first row's inverse stage has read its LDS
         fft_column<L, -1, true, false>(mylds, j, tw, load, nostore);
-        if (mine && rowok) {
-          const int off[2] = {lpad(tl), lpad(L - 1 - tl)};
-          switch (nv) {
-            case 1: oz_points_reg<1>(slds, CS, off, fkp, P, chr); break;
-            case 2: oz_points_reg<2>(slds, CS, off, fkp, P, chr); break;
-            case 3: oz_points_reg<3>(slds, CS, off, fkp, P, chr); break;
-            default: oz_points_reg<4>(slds, CS, off, fkp, P, chr); break;
+#pragma unroll
+        for (int k = 0; k < NP; ++k) {
+          if (mine[k] && rowok) {
+            const int jx = tl + k * nthr;
+            const int off[2] = {lpad(jx), lpad(L - 1 - jx)};
+            if (nv == 1)
+              oz_points_reg<1>(slds, CS, off, fkp[k], P, chr[k]);
+            else if (NVMAX == 2 || nv == 2)
+              oz_points_reg<2>(slds, CS, off, fkp[k], P, chr[k]);
+            else if constexpr (NVMAX == 4) {
+              if (nv == 3)
+                oz_points_reg<3>(slds, CS, off, fkp[k], P, chr[k]);
+              else
+                oz_points_reg<4>(slds, CS, off, fkp[k], P, chr[k]);
+            }
           }
         }
         __syncthreads();
@@ -296,7 +362,7 @@ __global__ void __launch_bounds__(512)
     asm volatile("" : "+s"(zero));
     const C *tw = twL + zero, *px = prex + zero;
     const bool rowok = r ? pair : live;
-    if (!kSlots && !rowok) break;  // as above
+    if ((!kSlots && !rowok) || (r && !paired)) break;  // as above
     const int y = r ? y1 : y0;
     const size_t rowoff = rowok ? ((size_t)m * P.ny + y) * L : 0;
     C *row = spec + (size_t)v * rowstride + rowoff;
@@ -314,10 +380,8 @@ __global__ void __launch_bounds__(512)
 
     // OZ at every k of the row, the mirror points (kx, -kx) together
     for (int jx = tl; rowok && jx < L / 2; jx += nthr) {
-      if constexpr (SHELL) {
-        const long ox = 2 * jx - L + 1;
-        const long sidx = (ox * ox + oy * oy + oz * oz - 3) >> 3;  // |k|^2 = (pi/L)^2 (8 sidx + 3)
-        oz_row<NVMAX>(slds, CS, jx, L, fkr, P, ChiTable<Re>{chitab + sidx * nv2});
+      if constexpr (CHI != RISM_CHI_SPLINE) {
+        oz_row<NVMAX>(slds, CS, jx, L, fkr, P, chi_row<L, CHI>(chitab, P, nv2, jx, yh, m));
       } else {
         const double ky = P.kfac[1] * ((double)y - (double)P.ny / 2.0 + 0.5);
         const double kz = P.kfac[2] * ((double)(m + P.nz / 2) - (double)P.nz / 2.0 + 0.5);
@@ -363,6 +427,26 @@ __global__ void k_chi_table(const double *__restrict__ knots, const double *__re
   for (int pw = 0; pw < nv2; ++pw) out[i * nv2 + pw] = X(pw);
 }
 
+// chi_vv at every point of the octant kx, ky, kz > 0 of a box with different
+// sides: |k| and the spline as the x pass evaluates them,
+// out[m][yh][pair][xh].
+__global__ void k_chi_octant(const double *__restrict__ knots, const double *__restrict__ coef,
+                             Params P, double *__restrict__ out) {
+  const int nxh = P.nx / 2, nyh = P.ny / 2;
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (size_t)nxh * nyh * (P.nz / 2)) return;
+  const int jx = (int)(i % nxh), y = (int)((i / nxh) % nyh), m = (int)(i / ((size_t)nxh * nyh));
+  const double ky = P.kfac[1] * ((double)y - (double)P.ny / 2.0 + 0.5);
+  const double kz = P.kfac[2] * ((double)(m + P.nz / 2) - (double)P.nz / 2.0 + 0.5);
+  const double kx = P.kfac[0] * ((double)jx - (double)P.nx / 2.0 + 0.5);
+  const double kk = sqrt(kx * kx + ky * ky + kz * kz);
+  const int ii = spline_interval(knots, P.np, P.x0, P.idk, kk);
+  const int nv2 = P.natv * P.natv;
+  const ChiSpline X{coef + (size_t)ii * 4 * nv2, kk - knots[ii], nv2};
+  double *row = out + (i / nxh) * nv2 * nxh + jx;
+  for (int pw = 0; pw < nv2; ++pw) row[(size_t)pw * nxh] = X(pw);
+}
+
 template <int L, class Re>
 static void launch_xoz(const Params &P, cx<Re> *spec, const cx<Re> *fkraw, const cx<Re> *twL,
                        const cx<Re> *prex, const double *knots, const double *coef,
@@ -370,12 +454,18 @@ static void launch_xoz(const Params &P, cx<Re> *spec, const cx<Re> *fkraw, const
   dim3 grid(P.ny, P.nz / 2, P.grp ? P.ngrp : 1);
   const int threads = P.natv * FftShape<L>::T;
   const size_t lds = (size_t)P.natv * FftShape<L>::CS * sizeof(cx<Re>);
-  // the OZ pass takes the rows in mirror pairs (y, ny-1-y), and short rows
-  // several pairs to a workgroup (row slots), so that it fills a wave
+  // the OZ pass takes the rows in mirror pairs (y, ny-1-y), one after the
+  // other, when the pairs are enough workgroups to fill the chip
+  const int ngrp = P.grp ? P.ngrp : 1;
+  // short rows: several to a workgroup (row slots), so that it fills a wave
   const int slots = (FftShape<L>::T >= 64 || threads >= 64) ? 1 : 64 / threads;
-  const dim3 pgrid(((P.ny + 1) / 2 + slots - 1) / slots, P.nz / 2, P.grp ? P.ngrp : 1);
   const int pthreads = slots * threads;
   const size_t plds = (size_t)slots * lds;
+  const long waves = ((pthreads + 63) / 64) * (long)((P.ny / 2 + slots - 1) / slots) *
+                     (P.nz / 2) * ngrp;
+  const int paired = waves >= kPairedWaves;
+  const int nrow = paired ? (P.ny + 1) / 2 : P.ny;
+  const dim3 pgrid((nrow + slots - 1) / slots, P.nz / 2, ngrp);
   if constexpr (sizeof(Re) == sizeof(double)) {
     if (P.mode == 1 || P.mode == 2) {
       if (P.mode == 1)
@@ -392,12 +482,23 @@ static void launch_xoz(const Params &P, cx<Re> *spec, const cx<Re> *fkraw, const
       (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)plds);
     hipLaunchKernelGGL(kern, pgrid, dim3(pthreads), plds, st, spec, fkraw, P, twL, prex, knots,
-                       coef, chitab);
+                       coef, chitab, paired);
   };
-  if (P.natv <= 4)
-    P.shell ? go(k_xpass_oz<L, 4, true, Re>) : go(k_xpass_oz<L, 4, false, Re>);
+  auto chi = [&](auto nvmax) {
+    constexpr int NVMAX = decltype(nvmax)::value;
+    if (P.shell == RISM_CHI_SHELL)
+      go(k_xpass_oz<L, NVMAX, RISM_CHI_SHELL, Re>);
+    else if (P.shell == RISM_CHI_OCTANT)
+      go(k_xpass_oz<L, NVMAX, RISM_CHI_OCTANT, Re>);
+    else  // the spline: one kernel for up to 4 sites
+      go(k_xpass_oz<L, (NVMAX < 4 ? 4 : NVMAX), RISM_CHI_SPLINE, Re>);
+  };
+  if (P.natv <= 2)
+    chi(std::integral_constant<int, 2>{});
+  else if (P.natv <= 4)
+    chi(std::integral_constant<int, 4>{});
   else
-    P.shell ? go(k_xpass_oz<L, 8, true, Re>) : go(k_xpass_oz<L, 8, false, Re>);
+    chi(std::integral_constant<int, 8>{});
 }
 int xoz_threads(int L, int natv) {
   switch (L) {
@@ -436,6 +537,13 @@ hipError_t run_chi_table(const double *knots, const double *coef, const Params &
                           double kscale, size_t nshell, double *out, hipStream_t st) {
   hipLaunchKernelGGL(k_chi_table, dim3((unsigned)((nshell + 255) / 256)), dim3(256), 0, st, knots,
                      coef, P, kscale, nshell, out);
+  return hipGetLastError();
+}
+hipError_t run_chi_octant(const double *knots, const double *coef, const Params &P, double *out,
+                          hipStream_t st) {
+  const size_t n = (size_t)(P.nx / 2) * (P.ny / 2) * (P.nz / 2);
+  hipLaunchKernelGGL(k_chi_octant, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, knots,
+                     coef, P, out);
   return hipGetLastError();
 }
 
