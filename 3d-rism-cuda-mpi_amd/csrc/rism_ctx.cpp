@@ -157,7 +157,6 @@ struct rism_ctx {
   std::vector<double> rho, qv, sigv, epsv;
   double temper = 0, xt = 0;
   int natu = 0;
-  std::vector<double> atoms_host;  // per atom record, rism::atom_stride(natv) doubles
   std::vector<double> usig, ueps, uq, uxyz;  // the solute as given (for .huv/.cuv headers)
   rism_opts opts{};
   // device: the FP64 level, and the FP32 level of a mixed-precision context
@@ -165,7 +164,11 @@ struct rism_ctx {
   Level<float> f;
   int prec = 0;  // level the loop runs at: 0 FP64, 1 FP32
   double *partial = nullptr, *tpartial = nullptr, *sums = nullptr, *scratch = nullptr;
-  double *atoms = nullptr, *knots = nullptr, *coef = nullptr, *chitab = nullptr;
+  // the solute as run_potential_r takes it: atoms sorted by type
+  double *atoms = nullptr, *tdata = nullptr;
+  int *trange = nullptr;
+  int ntype = 0;
+  double *knots = nullptr, *coef = nullptr, *chitab = nullptr;
   size_t nchitab = 0;  // doubles in chitab
   size_t zinv_blocks = 0;
   std::vector<void *> allocs;
@@ -415,6 +418,57 @@ int check_sizes(int nx, int ny, int nz, int natv) {
   if (natv > 8 || rism::xoz_threads(nx, natv) > 512)
     return rism::set_error(RISM_ERR_ARG, "natv must be <= 8 (and <= 4 for nx = 1024)");
   return RISM_OK;
+}
+
+// The solute's atoms sorted by type (equal sigma and epsilon), and the
+// Lennard-Jones coefficients of each type with every site (the mixing rules of
+// cal_LJ.cu:26-44; -l scales sigma).
+int make_solute(rism_ctx *c) {
+  const double lam1 = (c->opts.ad_switch == 1) ? c->opts.lambda : 1.0;
+  const int nv = c->natv, nu = c->natu;
+  // by bit pattern: a value that is no number is a type of its own
+  auto bits = [](double x) {
+    uint64_t b;
+    std::memcpy(&b, &x, sizeof(b));
+    return b;
+  };
+  std::map<std::pair<uint64_t, uint64_t>, int> types;
+  std::vector<int> type(nu), first;  // first: an atom of each type
+  for (int a = 0; a < nu; ++a) {
+    const auto it = types.emplace(std::make_pair(bits(c->usig[a]), bits(c->ueps[a])),
+                                  (int)types.size());
+    if (it.second) first.push_back(a);
+    type[a] = it.first->second;
+  }
+  const int nt = (int)types.size();
+  std::vector<int> range(nt + 1, 0);
+  for (int t : type) ++range[t + 1];
+  for (int t = 0; t < nt; ++t) range[t + 1] += range[t];
+  std::vector<int> at(range.begin(), range.end() - 1);
+  std::vector<double> atoms(4 * (size_t)std::max(nu, 1), 0.0);
+  for (int a = 0; a < nu; ++a) {
+    double *p = atoms.data() + 4 * (size_t)at[type[a]]++;
+    for (int d = 0; d < 3; ++d) p[d] = c->uxyz[3 * (size_t)a + d];
+    p[3] = c->uq[a];
+  }
+  std::vector<double> data((size_t)std::max(nt, 1) * (1 + 3 * nv), 0.0);
+  for (int t = 0; t < nt; ++t) {
+    double *p = data.data() + (size_t)t * (1 + 3 * nv);
+    for (int v = 0; v < nv; ++v) {  // cal_LJ.cu:33-44: sigma_uv, 4 eps_uv
+      const double su = (c->usig[first[t]] + c->sigv[v]) * 0.5 * lam1;
+      const double s2 = su * su, s6 = s2 * s2 * s2;
+      const double e4 = 4.0 * std::sqrt(c->ueps[first[t]] * c->epsv[v]);
+      p[0] = std::max(p[0], 4.0e-6 * s2);
+      p[1 + v] = s2;
+      p[1 + nv + v] = e4 * s6 * s6;
+      p[1 + 2 * nv + v] = e4 * s6;
+    }
+  }
+  c->ntype = nt;
+  int rc;
+  if ((rc = upload(c, &c->atoms, atoms))) return rc;
+  if ((rc = upload(c, &c->trange, range))) return rc;
+  return upload(c, &c->tdata, data);
 }
 
 void reset_an2(rism_ctx *c) {
@@ -1330,13 +1384,14 @@ int setup_enqueue(rism_ctx *c) {
   const int do_coul = c->opts.ad_switch != 1;  // cal_Coulomb.cu:23
   {
     KTime kt(c, RISM_K_POT);
-    HIPCHECK(rism::run_potential_r(c->atoms, c->natu, c->P, ikbt, ubeta, do_coul, c->d.u,
-                                   c->d.fr, c->st));
+    HIPCHECK(rism::run_potential_r(c->atoms, c->trange, c->tdata, c->ntype, c->P, ikbt, ubeta,
+                                   do_coul, c->d.u, c->d.fr, c->st));
   }
   if (do_coul && c->natu > 0) {
     KTime kt(c, RISM_K_FK);
-    HIPCHECK(rism::run_fk_half(c->atoms, c->natu, rism::atom_stride(c->natv), c->P, ubeta,
-                               c->d.fk, c->st));
+    // the spectrum's memory is free before the first step
+    HIPCHECK(rism::run_fk_half(c->atoms, c->natu, c->P, ubeta, c->d.spec,
+                               (size_t)c->natv * c->N / 2, c->d.fk, c->st));
   } else {
     HIPCHECK(hipMemsetAsync(c->d.fk, 0, sizeof(cplx) * (c->N / 2), c->st));
   }
@@ -1655,29 +1710,7 @@ rism_ctx *rism_create(const rism_grid *grid, const rism_solvent *solvent,
   c->P.clos = opts->closure;
   fill_params(c);
 
-  // solute table: cal_LJ.cu:26-40 mixing rules, -l scales sigma
-  const double lam1 = (opts->ad_switch == 1) ? opts->lambda : 1.0;
-  const int stride = rism::atom_stride(c->natv);
-  c->atoms_host.assign((size_t)(c->natu > 0 ? c->natu : 1) * stride, 0.0);
-  for (int a = 0; a < c->natu; ++a) {
-    double *p = c->atoms_host.data() + (size_t)a * stride;
-    p[0] = solute->xyz[3 * a];
-    p[1] = solute->xyz[3 * a + 1];
-    p[2] = solute->xyz[3 * a + 2];
-    p[3] = solute->q[a];
-    double rc2 = 0.0;
-    for (int v = 0; v < c->natv; ++v) {  // cal_LJ.cu:33-44: sigma_uv, 4 eps_uv
-      const double su = (solute->sig[a] + c->sigv[v]) * 0.5 * lam1;
-      const double s2 = su * su, s6 = s2 * s2 * s2;
-      const double e4 = 4.0 * std::sqrt(solute->eps[a] * c->epsv[v]);
-      p[5 + v] = s2;
-      p[5 + c->natv + v] = e4 * s6 * s6;
-      p[5 + 2 * c->natv + v] = e4 * s6;
-      rc2 = std::max(rc2, 4.0e-6 * s2);
-    }
-    p[4] = rc2;
-  }
-  if ((rc = upload(c, &c->atoms, c->atoms_host))) return fail(rc);
+  if ((rc = make_solute(c))) return fail(rc);
   if ((rc = make_tables(c, c->d.tb))) return fail(rc);
   if ((rc = make_chi(c, solvent))) return fail(rc);
 

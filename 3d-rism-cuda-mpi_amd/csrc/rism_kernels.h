@@ -86,10 +86,6 @@ struct HistUpdateT {
   int nh;
 };
 
-// doubles per solute atom record of the potential kernels: x, y, z, q,
-// rc2, sigma_uv^2[natv], 4 eps sigma^12 [natv], 4 eps sigma^6 [natv]
-inline __host__ __device__ int atom_stride(int natv) { return 5 + 3 * natv; }
-
 bool fft_length_supported(int L);
 // workgroups of the residual pass (hm: with the Anderson(m) sums)
 template <class Re>
@@ -184,10 +180,14 @@ hipError_t run_rebase_down(const double *x, const double *t0, float *out, size_t
                            hipStream_t st);
 // streaming copy of n doubles (n even): reads n, writes n
 hipError_t run_copy(const double *in, double *out, size_t n, hipStream_t st);
-hipError_t run_potential_r(const double *atoms, int natu, const Params &P, double ikbt,
-                           double ubeta, int do_coul, double *u, double *fr, hipStream_t st);
-hipError_t run_fk_half(const double *atoms, int natu, int astride, const Params &P,
-                       double ubeta, cplx *fkraw, hipStream_t st);
+// atoms: x, y, z, q each, sorted by type; type t: atoms [trange[t],
+// trange[t+1]) and 1 + 3 natv values in tdata (rism_kpot.hip)
+hipError_t run_potential_r(const double *atoms, const int *trange, const double *tdata, int ntype,
+                           const Params &P, double ikbt, double ubeta, int do_coul, double *u,
+                           double *fr, hipStream_t st);
+// work: nwork complex of scratch, at least nx/2 + ny + nz/2
+hipError_t run_fk_half(const double *atoms, int natu, const Params &P, double ubeta, cplx *work,
+                       size_t nwork, cplx *fkraw, hipStream_t st);
 hipError_t run_init_t(double *t, const double *fr, const Params &P, size_t N, hipStream_t st);
 template <class Re>
 hipError_t run_fields(const Re *t, const Re *u, const Re *R, const Params &P, size_t n,

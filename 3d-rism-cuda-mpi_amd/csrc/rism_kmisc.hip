@@ -1,5 +1,5 @@
-// rism_kmisc.hip -- FP64 reductions, the AN2 update, set-up potentials,
-// k-space Coulomb, initial t, derived fields and thermodynamic partial sums.
+// rism_kmisc.hip -- FP64 reductions, the AN2 update, initial t, derived fields,
+// per-atom and thermodynamic partial sums.
 #include <algorithm>
 
 #include "rism_common.h"
@@ -394,148 +394,6 @@ __global__ void k_convert(const From *__restrict__ in, To *__restrict__ out, siz
 }
 
 // ---------------------------------------------------------------------------
-// set-up: potentials (cal_LJ.cu:56-81, cal_Coulomb.cu:40-62, cal_potential.cu:39-43)
-// ---------------------------------------------------------------------------
-// Each thread owns PX consecutive x points of one (y, z) line and a group of
-// G <= 8 solvent sites starting at v0; solute atoms stream through LDS in
-// tiles of ATILE records (atom_stride(natv) doubles: x, y, z, q, rc2,
-// sigma_uv^2[natv], A[natv] = 4 eps sigma^12, B[natv] = 4 eps sigma^6).
-// 4 eps (s^-12 - s^-6) with s^2 = r^2 / sigma^2 is A r^-12 - B r^-6, so the
-// powers of 1/r are formed once per pair and each site costs two FMAs.  The
-// reference's floor s^2 >= 4e-6 (cal_LJ.cu:11-12) can only bind when
-// r^2 < rc2 = 4e-6 max_v sigma_uv^2; those (rare) pairs take the clamped form.
-// Outputs u[v] = beta sum LJ + q_v de, and fr (first group).
-// 1/r comes from the v_rsq_f64 seed refined by two Newton steps, so the pair
-// loop has no FP64 division or square root.
-constexpr int PX = 4;
-constexpr int ATILE = 256;
-
-// 1/sqrt(x) in FP64: the hardware estimate (relative error up to 5.2e-8 on
-// this part) and one third-order (Halley-type) correction, y (1 + e/2 +
-// 3e^2/8) with e = 1 - x y^2: measured within 1.4e-16 relative over
-// x in [1e-4, 1e6], against 2.4e-16 for two Newton steps, in 5 operations
-// instead of 7
-__device__ __forceinline__ double rsq_nr(double x) {
-  const double y = __builtin_amdgcn_rsq(x);
-  const double e = fma(-x * y, y, 1.0);
-  return fma(y * e, fma(e, 0.375, 0.5), y);
-}
-
-// 1/x in FP64 for the rare clamped pairs: the hardware estimate and two
-// Newton steps, within an ulp of the IEEE quotient (with the IEEE division
-// sequence the 4-site pair loop spills at the four-wave register limit)
-__device__ __forceinline__ double rcp_nr(double x) {
-  double y = __builtin_amdgcn_rcp(x);
-  y = fma(fma(-x, y, 1.0), y, y);
-  return fma(fma(-x, y, 1.0), y, y);
-}
-
-// Up to 4 sites per launch the pair loop fits 128 VGPRs without spilling and
-// runs four waves per SIMD instead of the three its unconstrained 138 VGPRs
-// allow (512^3, 12877 atoms, 4 sites: 1.88 -> 1.65 s); 5-8 sites would
-// spill at that limit and keep the default.
-template <int G>
-constexpr int potential_waves_per_eu() {
-  return G <= 4 ? 4 : 1;
-}
-
-template <int G, bool COUL>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(potential_waves_per_eu<G>())))
-    k_potential_r(const double *__restrict__ atoms, int natu, int v0, Params P, double ikbt,
-                  double ubeta, int write_fr, double *__restrict__ u,
-                  double *__restrict__ fr) {
-  extern __shared__ double sa[];
-  const int nv = P.natv;
-  const int stride = atom_stride(nv);
-  const int nxq = (P.nx + PX - 1) / PX;
-  const size_t lines = (size_t)P.ny * P.nz;
-  const size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const bool active = gid < lines * (size_t)nxq;
-  const int xq = active ? (int)(gid % nxq) : 0;
-  const size_t line = active ? gid / nxq : 0;
-  const int y = (int)(line % P.ny), z = (int)(line / P.ny);
-  const double ry = (double)(y - P.ny / 2) * P.dr[1];
-  const double rz = (double)(z - P.nz / 2) * P.dr[2];
-  double rx[PX];
-#pragma unroll
-  for (int p = 0; p < PX; ++p) rx[p] = (double)(xq * PX + p - P.nx / 2) * P.dr[0];
-  double lj[PX][G];
-  double de[PX], ff[PX];
-#pragma unroll
-  for (int p = 0; p < PX; ++p) {
-    de[p] = 0.0;
-    ff[p] = 0.0;
-#pragma unroll
-    for (int w = 0; w < G; ++w) lj[p][w] = 0.0;
-  }
-  constexpr double icut2 = 1.0 / (2.0e-3 * 2.0e-3);  // s^2 >= 4e-6 (cal_LJ.cu:11-12)
-  for (int a0 = 0; a0 < natu; a0 += ATILE) {
-    const int na = min(ATILE, natu - a0);
-    __syncthreads();
-    for (int i = threadIdx.x; i < na * stride; i += blockDim.x)
-      sa[i] = atoms[(size_t)a0 * stride + i];
-    __syncthreads();
-    for (int a = 0; a < na; ++a) {
-      const double *at = sa + a * stride;
-      const double ax = at[0], ay = at[1], az = at[2], aq = at[3], rc2 = at[4];
-      double A[G], B[G];
-#pragma unroll
-      for (int w = 0; w < G; ++w) {
-        A[w] = at[5 + nv + v0 + w];
-        B[w] = at[5 + 2 * nv + v0 + w];
-      }
-      const double dy = ry - ay, dz = rz - az;
-      const double dyz = dy * dy + dz * dz;
-#pragma unroll
-      for (int p = 0; p < PX; ++p) {
-        const double dx = rx[p] - ax;
-        const double r2 = dx * dx + dyz;
-        const double ir = rsq_nr(r2);  // NaN at r2 = 0: both uses below handle it
-        const double ir2 = ir * ir;
-        if (r2 >= rc2) {
-          // A r^-12 - B r^-6 = r^-6 (A r^-6 - B)
-          const double ir6 = ir2 * ir2 * ir2;
-#pragma unroll
-          for (int w = 0; w < G; ++w) lj[p][w] = fma(fma(A[w], ir6, -B[w]), ir6, lj[p][w]);
-        } else {
-#pragma unroll
-          for (int w = 0; w < G; ++w) {
-            const double sg2 = at[5 + v0 + w];
-            const double e4 = B[w] * rcp_nr(sg2 * sg2 * sg2);
-            const double s2 = fmin(sg2 * ir2, icut2);  // fmin drops the NaN of r = 0
-            const double s6 = s2 * s2 * s2;
-            lj[p][w] += e4 * s6 * (s6 - 1.0);
-          }
-        }
-        if constexpr (COUL) {
-          if (r2 >= 1.0e-10) {  // r >= 1e-5
-            const double qr = aq * ir;
-            de[p] += qr;
-            // 1 - e^{-r} rounds to exactly 1 in FP64 once r > 37.5
-            ff[p] += (r2 < 38.0 * 38.0) ? qr * (1.0 - exp(-(r2 * ir))) : qr;
-          } else {
-            ff[p] += aq;
-          }
-        }
-      }
-    }
-  }
-  if (!active) return;
-  const size_t N = (size_t)P.nx * P.ny * P.nz;
-  const size_t rowbase = line * P.nx;
-#pragma unroll
-  for (int p = 0; p < PX; ++p) {
-    const int x = xq * PX + p;
-    if (x >= P.nx) break;
-    const double e = de[p] * ubeta;
-#pragma unroll
-    for (int w = 0; w < G; ++w)
-      u[(size_t)(v0 + w) * N + rowbase + x] = lj[p][w] * ikbt + P.qv[v0 + w] * e;
-    if (write_fr) fr[rowbase + x] = ff[p] * ubeta;
-  }
-}
-
-// ---------------------------------------------------------------------------
 // per-atom integrals of the converged g (cal_grad.cu:44-90, cal_euv.cu:30-70,
 // cal_ad1.cu:40-80, cal_ad2.cu:40-75): for each solute atom u, sums over the
 // grid points r with |r - r_u| >= sigma_uv / 2 (sigma_uv lambda / 2 for ad1)
@@ -647,85 +505,6 @@ __global__ void __launch_bounds__(256)
   } else {
 #pragma unroll
     for (int k = 0; k < (int)(sizeof(acc) / sizeof(double)); ++k) out[k] = acc[k];
-  }
-}
-
-// fk on the half spectrum (cal_Coulomb.cu:65-79, 90-95), stored raw:
-// fkraw = conj(phi(k)) fk, phi(k) = -i (-1)^(nx/2 + ny/2 + jx + jy + m).
-// Each thread owns FKP consecutive jx of one (jy, m) row; e^{-i kx x_u} is
-// advanced along the row by the recurrence e^{-i (kx + dkx) x_u} =
-// e^{-i kx x_u} e^{-i dkx x_u}.
-constexpr int FKP = 16;
-
-__global__ void __launch_bounds__(256)
-    k_fk_half(const double *__restrict__ atoms, int natu, int astride, Params P, double ubeta,
-              cplx *__restrict__ fkraw) {
-  // per atom: x, y, z, q and the x-phase step e^{-i dkx x} (cos, sin), formed
-  // once per atom by the thread that stages it
-  __shared__ double sa[ATILE * 6];
-  const int M = P.nz / 2;
-  const int nxq = (P.nx + FKP - 1) / FKP;
-  const size_t rows = (size_t)P.ny * M;
-  const size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const bool active = gid < rows * (size_t)nxq;
-  const int xq = active ? (int)(gid % nxq) : 0;
-  const size_t row = active ? gid / nxq : 0;
-  const int jy = (int)(row % P.ny), m = (int)(row / P.ny);
-  const int jx0 = xq * FKP;
-  const double kx0 = P.kfac[0] * ((double)jx0 - (double)P.nx / 2.0 + 0.5);
-  const double ky = P.kfac[1] * ((double)jy - (double)P.ny / 2.0 + 0.5);
-  const double kz = P.kfac[2] * ((double)(m + P.nz / 2) - (double)P.nz / 2.0 + 0.5);
-  const double dkx = P.kfac[0];
-  double re[FKP], im[FKP];
-#pragma unroll
-  for (int p = 0; p < FKP; ++p) re[p] = im[p] = 0.0;
-  for (int a0 = 0; a0 < natu; a0 += ATILE) {
-    const int na = min(ATILE, natu - a0);
-    __syncthreads();
-    for (int i = threadIdx.x; i < na; i += blockDim.x) {
-      const double *src = atoms + (size_t)(a0 + i) * astride;
-      double dsn, dcs;
-      sincos(dkx * src[0], &dsn, &dcs);
-      sa[6 * i] = src[0];
-      sa[6 * i + 1] = src[1];
-      sa[6 * i + 2] = src[2];
-      sa[6 * i + 3] = src[3];
-      sa[6 * i + 4] = dcs;
-      sa[6 * i + 5] = dsn;
-    }
-    __syncthreads();
-    for (int a = 0; a < na; ++a) {
-      const double ax = sa[6 * a], ay = sa[6 * a + 1], az = sa[6 * a + 2], aq = sa[6 * a + 3];
-      const double dcs = sa[6 * a + 4], dsn = sa[6 * a + 5];
-      double sn, cs;
-      sincos(kx0 * ax + ky * ay + kz * az, &sn, &cs);
-      // e = cos - i sin; step = dcs - i dsn
-      double er = cs, ei = -sn;
-#pragma unroll
-      for (int p = 0; p < FKP; ++p) {
-        re[p] += aq * er;
-        im[p] += aq * ei;
-        const double nr = er * dcs + ei * dsn;
-        const double ni = ei * dcs - er * dsn;
-        er = nr;
-        ei = ni;
-      }
-    }
-  }
-  if (!active) return;
-  const int sgn0 = ((P.nx / 2 + P.ny / 2 + jy + m) & 1) ? -1 : 1;
-#pragma unroll
-  for (int p = 0; p < FKP; ++p) {
-    const int jx = jx0 + p;
-    if (jx >= P.nx) break;
-    const double kx = P.kfac[0] * ((double)jx - (double)P.nx / 2.0 + 0.5);
-    const double rk2 = kx * kx + ky * ky + kz * kz;
-    const double rk4i = 1.0 / (rk2 * (rk2 + 1.0));
-    const double f = 4.0 * M_PI * rk4i * ubeta;
-    const double fre = f * re[p], fim = f * im[p];
-    // conj(phi) = i * s
-    const double s = ((jx & 1) ? -sgn0 : sgn0);
-    fkraw[row * P.nx + jx] = mk(-s * fim, s * fre);
   }
 }
 
@@ -944,41 +723,6 @@ hipError_t run_rebase_down(const double *x, const double *t0, float *out, size_t
   return hipGetLastError();
 }
 template hipError_t run_convert<float, double>(const float *, double *, size_t, hipStream_t);
-
-hipError_t run_potential_r(const double *atoms, int natu, const Params &P, double ikbt,
-                           double ubeta, int do_coul, double *u, double *fr, hipStream_t st) {
-  const size_t nth = (size_t)P.ny * P.nz * ((P.nx + PX - 1) / PX);
-  const size_t lds = (size_t)ATILE * atom_stride(P.natv) * sizeof(double);
-  const dim3 grid(nblk(nth, 256)), block(256);
-  for (int v0 = 0; v0 < P.natv; v0 += 8) {
-    const int g = min(8, P.natv - v0);
-    const int wf = v0 == 0;
-    switch (g) {
-#define G_CASE(n)                                                                              \
-  case n:                                                                                      \
-    if (do_coul)                                                                               \
-      hipLaunchKernelGGL((k_potential_r<n, true>), grid, block, lds, st, atoms, natu, v0, P,   \
-                         ikbt, ubeta, wf, u, fr);                                              \
-    else                                                                                       \
-      hipLaunchKernelGGL((k_potential_r<n, false>), grid, block, lds, st, atoms, natu, v0, P,  \
-                         ikbt, ubeta, wf, u, fr);                                              \
-    break;
-      G_CASE(1) G_CASE(2) G_CASE(3) G_CASE(4) G_CASE(5) G_CASE(6) G_CASE(7) G_CASE(8)
-#undef G_CASE
-    }
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
-}
-
-hipError_t run_fk_half(const double *atoms, int natu, int astride, const Params &P,
-                       double ubeta, cplx *fkraw, hipStream_t st) {
-  const size_t nth = (size_t)P.ny * (P.nz / 2) * ((P.nx + FKP - 1) / FKP);
-  hipLaunchKernelGGL(k_fk_half, dim3(nblk(nth, 256)), dim3(256), 0, st, atoms, natu, astride, P,
-                     ubeta, fkraw);
-  return hipGetLastError();
-}
 
 hipError_t run_init_t(double *t, const double *fr, const Params &P, size_t N, hipStream_t st) {
   hipLaunchKernelGGL(k_init_t, dim3(nblk(N * P.natv, 256)), dim3(256), 0, st, t, fr, P, N);
