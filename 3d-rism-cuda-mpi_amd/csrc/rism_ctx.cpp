@@ -644,7 +644,6 @@ int calc_step(rism_ctx *c, double *rms, bool lin = false, double tol = -1.0) {
     HIPCHECK(rism::run_y(P, L.spec, +1, L.tb.twy, L.tb.prey, c->st));
   }
   const bool andm = c->opts.anderson_m > 0;
-  const int W = andm ? kSumWidth : 6;
   Re *Rout = andm ? L.Rb[c->cur_rb] : L.R[c->iR_cur];
   {
     KTime kt(c, RISM_K_ZINV);
@@ -663,20 +662,19 @@ int calc_step(rism_ctx *c, double *rms, bool lin = false, double tol = -1.0) {
   const size_t nb = rism::zinv_num_blocks<Re>(P, andm ? 1 : 0) / c->natv;
   {
     KTime kt(c, RISM_K_REDUCE);
-    HIPCHECK(rism::run_reduce_cols(c->partial, nb, W, c->natv, c->sums, P.done, c->st));
+    double *hist = c->async ? c->rms_hist : nullptr;
+    int *flag = c->async ? c->dflag : nullptr;
     if (andm) {
       int rb[RISM_MAX_HIST];
       const int nh = (int)c->hist.size();
       for (int p = 0; p < nh; ++p) rb[p] = c->hist[p].rb;
-      HIPCHECK(rism::run_andm_finish(c->sums, c->rho_dev, c->natv, c->N, tol, W, c->dD,
-                                     c->opts.anderson_m + 1, c->cur_rb, rb, nh, c->count == 0,
-                                     c->xcoef, c->scal, c->async ? c->rms_hist : nullptr,
-                                     c->async ? c->dflag : nullptr, c->st));
+      HIPCHECK(rism::run_andm_finish(c->partial, nb, c->sums, c->rho_dev, c->natv, c->N, tol,
+                                     kSumWidth, c->dD, c->opts.anderson_m + 1, c->cur_rb, rb, nh,
+                                     c->count == 0, c->xcoef, c->scal, hist, flag, c->st));
     } else {
-      HIPCHECK(rism::run_step_finish(c->sums, c->rho_dev, c->natv, c->N, tol,
-                                     c->count == 0, c->opts.an2_mp, c->binary, c->scal,
-                                     c->async ? c->rms_hist : nullptr,
-                                     c->async ? c->dflag : nullptr, c->st));
+      HIPCHECK(rism::run_step_finish(c->partial, nb, c->sums, c->rho_dev, c->natv, c->N, tol,
+                                     c->count == 0, c->opts.an2_mp, c->binary, c->scal, hist,
+                                     flag, c->st));
     }
   }
   c->iT_last = c->iT_cur;
@@ -1242,10 +1240,9 @@ int group_step(GroupRun &g) {
                           (const double *)nullptr, c->partial, L.tb.twz, L.tb.zpre, L.tb.zpost,
                           ix.count == 0, st));
   const size_t nb = rism::zinv_num_blocks<double>(P, 0) / c->natv;
-  HIPCHECK(rism::run_reduce_cols(c->partial, nb, 6, c->natv, c->sums, nullptr, st, tab, P.ngrp));
-  HIPCHECK(rism::run_step_finish(c->sums, c->rho_dev, c->natv, c->N, g.tol, ix.count == 0,
-                                 c->opts.an2_mp, ix.b, c->scal, c->rms_hist, c->dflag, st, tab,
-                                 P.ngrp));
+  HIPCHECK(rism::run_step_finish(c->partial, nb, c->sums, c->rho_dev, c->natv, c->N, g.tol,
+                                 ix.count == 0, c->opts.an2_mp, ix.b, c->scal, c->rms_hist,
+                                 c->dflag, st, tab, P.ngrp));
   const size_t nn = c->N * c->natv;
   if (ix.count > 0) {
     HIPCHECK(rism::run_an2_picard(L.T[1 - ix.iT], L.T[ix.iT], L.R[ix.iR], L.Pslot[ix.b],

@@ -131,31 +131,33 @@ template <class Re>
 hipError_t run_andm_update(Re *tnew, const Re *t, const Re *R, const HistUpdateT<Re> &H, Re *Pb,
                            const double *xcoef, double beta, size_t n, const int *done,
                            hipStream_t st);
-// End of an Anderson(m) step on the device: rms, flags and rms_hist as
-// run_step_finish (done may be null); the dots of the residual in buffer
-// `cur` with itself and the history buffers rb[0..nh) (oldest first) into
-// D[m1][m1]; when mixing, the nh coefficients into xcoef.  sums: [site][width]
-// FP64, R.R then R.R_p.
-hipError_t run_andm_finish(const double *sums, const double *rho, int natv, size_t N, double tol,
-                           int width, double *D, int m1, int cur, const int *rb, int nh,
-                           int mixing, double *xcoef, double *scal, double *rms_hist, int *done,
-                           hipStream_t st);
 // nsets consecutive blocks of nrow x width partial sums -> nsets x width
 hipError_t run_reduce_cols(const double *in, size_t nrow, int width, int nsets, double *out,
                            const int *done, hipStream_t st, const GroupPtrs *grp = nullptr,
                            int ngrp = 0);
 // End of one AN2 step on the device (cal_rms.cu:20-24 and, when the next
-// update mixes, cal_theta + leg of anderson.cu:81-130): from the per-site
-// sums (6 per site) it writes scal = {rms, x0, x1, s1, s2}.  With a flag
-// array done = {state, step, count} it also counts the step (count + 1),
-// writes rms_hist[step] and, when rms <= tol or rms is not finite, sets
-// state to 1 or 2 and step; no argument depends on the step number, so a
-// run of steps can be captured once and replayed.  binary: the slot the
-// next update retires.
-hipError_t run_step_finish(const double *sums, const double *rho, int natv, size_t N,
-                           double tol, int mixing, double mp, int binary, double *scal,
-                           double *rms_hist, int *done, hipStream_t st,
+// update mixes, cal_theta + leg of anderson.cu:81-130): from the residual
+// pass's partial sums (natv blocks of nrow rows of 6; sums: scratch for 6 per
+// site) it writes scal = {rms, x0, x1, s1, s2}.  With a flag array done =
+// {state, step, count} it also counts the step (count + 1), writes
+// rms_hist[step] and, when rms <= tol or rms is not finite, sets state to 1 or
+// 2 and step; no argument depends on the step number, so a run of steps can
+// be captured once and replayed.  binary: the slot the next update retires.
+hipError_t run_step_finish(const double *partial, size_t nrow, double *sums, const double *rho,
+                           int natv, size_t N, double tol, int mixing, double mp, int binary,
+                           double *scal, double *rms_hist, int *done, hipStream_t st,
                            const GroupPtrs *grp = nullptr, int ngrp = 0);
+// End of an Anderson(m) step on the device: rms, flags and rms_hist as
+// run_step_finish (done may be null); the dots of the residual in buffer
+// `cur` with itself and the history buffers rb[0..nh) (oldest first) into
+// D[m1][m1]; when mixing, the nh coefficients into xcoef.  partial: natv
+// blocks of nrow rows of width = 1 + RISM_MAX_HIST sums, R.R then R.R_p; sums:
+// scratch for width per site.
+hipError_t run_andm_finish(const double *partial, size_t nrow, double *sums, const double *rho,
+                           int natv, size_t N, double tol, int width, double *D, int m1, int cur,
+                           const int *rb, int nh, int mixing, double *xcoef, double *scal,
+                           double *rms_hist, int *done, hipStream_t st);
+// Pb (may be null) receives t + m R
 template <class Re>
 hipError_t run_an2_picard(Re *tnew, const Re *t, const Re *R, Re *Pb, double m, size_t n,
                           const int *done, hipStream_t st, const GroupPtrs *grp = nullptr,

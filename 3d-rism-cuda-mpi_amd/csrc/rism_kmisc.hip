@@ -154,40 +154,63 @@ __global__ void k_an2_update(V16<Re> *__restrict__ tnew, const V16<Re> *__restri
   st_nt(Pb + i, q);
 }
 
-// End of a step: rms (cal_rms.cu:20-24), convergence / divergence flag
-// (iterate.cu:50-57) and the AN2 mixing coefficients for the next update
-// (cal_theta anderson.cu:81-102 with the rho^-1 weights, leg()'s Gaussian
-// elimination without pivoting anderson.cu:105-130, the mp shift
-// anderson.cu:66-67).  One thread; the sums are 6 doubles per site.
-__global__ void k_step_finish(const double *__restrict__ sums, const double *__restrict__ rho,
-                              int natv, size_t N, double tol, int mixing, double mp, int binary,
-                              double *__restrict__ scal, double *__restrict__ rms_hist,
-                              int *__restrict__ done, const GroupPtrs *grp) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  if (grp) {
-    const GroupPtrs &g = grp[blockIdx.z];
-    sums = global_ptr<const double>(g.sums);
-    scal = global_ptr<double>(g.scal);
-    rms_hist = global_ptr<double>(g.rms_hist);
-    done = global_ptr<int>(g.done);
+// End of a step in one workgroup per context: the column sums of the residual
+// pass's partial sums, rms (cal_rms.cu:20-24), the convergence / divergence flag
+// (iterate.cu:50-57) and the mixing coefficients for the next update.
+// in: natv consecutive blocks of nrow rows of W sums.  Up to kOneGroupSums of
+// them are read here by one workgroup; more are reduced by k_reduce_cols first
+// and arrive as one row per site.  One kernel against the two: 64^3, 2 sites
+// (3072 sums) 4.4 against 4.0 + 3.0 us and a launch; 144 x 160 x 128, 4 sites
+// (34560) 8.1 against 4.8 + 4.6; 256^3, 4 sites (98304) 19.6 against 9.4 + 4.5.
+constexpr size_t kOneGroupSums = 3 << 14;
+constexpr int kEndThreads = 1024;
+
+// Sums into sh[v W + k] (v < natv, k < W): a thread keeps one column (of one
+// site) and every rp-th row, Kahan-compensated, then a tree over the rows.
+__device__ __forceinline__ void column_sums(const double *__restrict__ in, size_t nrow, int W,
+                                            int natv, double *sh) {
+  const int nt = blockDim.x, cols = natv * W;
+  const int rp = max(1, nt / cols);  // rows side by side
+  const int t = threadIdx.x, row = t / cols, col = t % cols;
+  const bool mine = row < rp;
+  double a = 0.0, comp = 0.0;
+  if (mine) {
+    const double *p = in + ((size_t)(col / W) * nrow) * W + col % W;
+    auto add = [&](double x) {
+      const double yv = x - comp;
+      const double tv = a + yv;
+      comp = (tv - a) - yv;
+      a = tv;
+    };
+    size_t r = row;
+    for (; r + 3 * rp < nrow; r += 4 * rp) {  // four loads in flight
+      const double x0 = p[r * W], x1 = p[(r + rp) * W], x2 = p[(r + 2 * rp) * W],
+                   x3 = p[(r + 3 * rp) * W];
+      add(x0);
+      add(x1);
+      add(x2);
+      add(x3);
+    }
+    for (; r < nrow; r += rp) add(p[r * W]);
+    sh[t] = a;
   }
-  if (done && done[0]) return;
+  __syncthreads();
+  for (int n = rp; n > 1;) {
+    const int h = (n + 1) / 2;
+    if (mine && row + h < n) sh[t] += sh[t + h * cols];
+    n = h;
+    __syncthreads();
+  }
+}
+
+// rms, its history and the flags: done = {state, step, count}
+__device__ __forceinline__ void step_record(double ss, int natv, size_t N, double tol,
+                                            double *scal, double *rms_hist, int *done) {
   // step number: done[2] counts the finished steps of the run
   int step = 0;
   if (done) {
     step = done[2] + 1;
     done[2] = step;
-  }
-  double ss = 0.0, cc0 = 0.0, cc1 = 0.0, a0 = 0.0, a1 = 0.0, a3 = 0.0;
-  for (int v = 0; v < natv; ++v) {
-    const double *s = sums + 6 * v;
-    const double ir = 1.0 / rho[v];
-    ss += s[0];
-    cc0 += s[1] * ir;
-    cc1 += s[2] * ir;
-    a0 += s[3] * ir;
-    a1 += s[4] * ir;
-    a3 += s[5] * ir;
   }
   const double rms = sqrt(ss / ((double)N * natv));
   scal[0] = rms;
@@ -201,6 +224,39 @@ __global__ void k_step_finish(const double *__restrict__ sums, const double *__r
       done[1] = step;
     }
   }
+}
+
+// AN2: the two-slot system (cal_theta anderson.cu:81-102 with the rho^-1
+// weights, leg()'s Gaussian elimination without pivoting anderson.cu:105-130,
+// the mp shift anderson.cu:66-67).
+__global__ void __launch_bounds__(kEndThreads)
+    k_step_finish(const double *__restrict__ in, size_t nrow, const double *__restrict__ rho,
+                  int natv, size_t N, double tol, int mixing, double mp, int binary,
+                  double *__restrict__ scal, double *__restrict__ rms_hist,
+                  int *__restrict__ done, const GroupPtrs *grp, int reduced) {
+  __shared__ double sums[kEndThreads];
+  if (grp) {
+    const GroupPtrs &g = grp[blockIdx.z];
+    in = reduced ? global_ptr<const double>(g.sums) : global_ptr<const double>(g.partial);
+    scal = global_ptr<double>(g.scal);
+    rms_hist = global_ptr<double>(g.rms_hist);
+    done = global_ptr<int>(g.done);
+  }
+  if (done && done[0]) return;
+  column_sums(in, nrow, 6, natv, sums);
+  if (threadIdx.x != 0) return;
+  double ss = 0.0, cc0 = 0.0, cc1 = 0.0, a0 = 0.0, a1 = 0.0, a3 = 0.0;
+  for (int v = 0; v < natv; ++v) {
+    const double *s = sums + 6 * v;
+    const double ir = 1.0 / rho[v];
+    ss += s[0];
+    cc0 += s[1] * ir;
+    cc1 += s[2] * ir;
+    a0 += s[3] * ir;
+    a1 += s[4] * ir;
+    a3 += s[5] * ir;
+  }
+  step_record(ss, natv, N, tol, scal, rms_hist, done);
   if (mixing) {
     const double a2 = a1;
     double b1 = a1, b3 = a3, c0 = cc0, c1 = cc1;
@@ -230,107 +286,131 @@ __global__ void k_step_finish(const double *__restrict__ sums, const double *__r
 // unit diagonal, Gaussian elimination with partial pivoting; when a pivot
 // falls below 1e-12 (or a diagonal is not positive) the oldest entry is left
 // out and the solve repeated.  th (zeros for entries left out) goes to
-// xcoef[0..nh).  One thread, FP64; W = 1 + RISM_MAX_HIST sums per site.
+// xcoef[0..nh).  FP64; W = 1 + RISM_MAX_HIST sums per site.
+// The first wave holds the 16 x 16 system in registers, lane l row l & 15 and
+// the four columns from 4 (l >> 4), and exchanges through shuffles (one thread
+// with its arrays in scratch memory took 101 us at m = 10, this 14).
 // ---------------------------------------------------------------------------
 struct AndmHist {
   int rb[RISM_MAX_HIST];
   int nh;
 };
+static_assert(RISM_MAX_HIST == 16, "the wave solve holds 16 rows");
 
-__global__ void k_andm_finish(const double *__restrict__ sums, const double *__restrict__ rho,
-                              int natv, size_t N, double tol, int W, double *__restrict__ D,
-                              int m1, int cur, AndmHist H, int mixing,
-                              double *__restrict__ xcoef, double *__restrict__ scal,
-                              double *__restrict__ rms_hist, int *__restrict__ done) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// element q & 3 of the four columns of a lane
+__device__ __forceinline__ double pick4(const double (&g)[4], int q) {
+  const double a = (q & 1) ? g[1] : g[0], b = (q & 1) ? g[3] : g[2];
+  return (q & 2) ? b : a;
+}
+
+__global__ void __launch_bounds__(kEndThreads)
+    k_andm_finish(const double *__restrict__ in, size_t nrow, const double *__restrict__ rho,
+                  int natv, size_t N, double tol, int W, double *__restrict__ D, int m1, int cur,
+                  AndmHist H, int mixing, double *__restrict__ xcoef, double *__restrict__ scal,
+                  double *__restrict__ rms_hist, int *__restrict__ done) {
+  __shared__ double sums[kEndThreads];
+  __shared__ double dots[1 + RISM_MAX_HIST];  // of R with itself and the history
+  __shared__ int rb[RISM_MAX_HIST];
   if (done && done[0]) return;
-  int step = 0;
-  if (done) {
-    step = done[2] + 1;
-    done[2] = step;
+  column_sums(in, nrow, W, natv, sums);
+  const int lane = threadIdx.x, nh = H.nh;
+  if (lane < RISM_MAX_HIST) {
+#pragma unroll
+    for (int p = 0; p < RISM_MAX_HIST; ++p)
+      if (p == lane) rb[p] = H.rb[p];
   }
-  double ss = 0.0;
-  for (int v = 0; v < natv; ++v) ss += sums[W * v];
-  const double rms = sqrt(ss / ((double)N * natv));  // cal_rms.cu:24
-  scal[0] = rms;
-  if (rms_hist) rms_hist[step] = rms;
-  if (done) {
-    if (!isfinite(rms)) {
-      done[0] = 2;
-      done[1] = step;
-    } else if (rms <= tol) {
-      done[0] = 1;
-      done[1] = step;
-    }
-  }
-  // weighted dots <R, R> and <R, R_p>, weights 1 / rho_v (anderson.cu:37-39)
-  auto wdot = [&](int k) {
+  if (lane <= RISM_MAX_HIST) {
+    // weighted dots, weights 1 / rho_v (anderson.cu:37-39)
     double a = 0.0;
-    for (int v = 0; v < natv; ++v) a += sums[W * v + k] / rho[v];
-    return a;
-  };
-  D[(size_t)cur * m1 + cur] = wdot(0);
-  for (int p = 0; p < H.nh; ++p) {
-    const int bb = H.rb[p];
-    D[(size_t)cur * m1 + bb] = D[(size_t)bb * m1 + cur] = wdot(1 + p);
+    if (lane <= nh)
+      for (int v = 0; v < natv; ++v) a += sums[W * v + lane] / rho[v];
+    dots[lane] = a;
   }
-  if (!mixing) return;
-  const int nh = H.nh;
-  for (int p = 0; p < nh; ++p) xcoef[p] = 0.0;
-  const double rr = D[(size_t)cur * m1 + cur];
-  double G[RISM_MAX_HIST][RISM_MAX_HIST], b[RISM_MAX_HIST], sc[RISM_MAX_HIST], x[RISM_MAX_HIST];
+  __syncthreads();
+  if (lane >= 64) return;
+  if (lane == 0) {
+    double ss = 0.0;
+    for (int v = 0; v < natv; ++v) ss += sums[W * v];
+    step_record(ss, natv, N, tol, scal, rms_hist, done);
+    D[(size_t)cur * m1 + cur] = dots[0];
+  }
+  if (lane < nh) {
+    D[(size_t)cur * m1 + rb[lane]] = dots[1 + lane];
+    D[(size_t)rb[lane] * m1 + cur] = dots[1 + lane];
+  }
+  if (!mixing || nh == 0) return;
+  const int r = lane & 15, h = lane >> 4;
+  const double rr = dots[0];
+  double th = 0.0;  // the coefficient of entry r
   for (int first = 0; first < nh; ++first) {
     const int k = nh - first;
+    const bool in_r = r < k;
+    const double dp = in_r ? dots[1 + first + r] : 0.0;
+    double g[4], b = rr - dp;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int q = 4 * h + c;
+      // dots among older residuals: entries of D that no lane writes here
+      g[c] = (in_r && q < k) ? rr - dp - dots[1 + first + q] +
+                                   D[(size_t)rb[first + r] * m1 + rb[first + q]]
+                             : 0.0;
+    }
+    const double diag = __shfl(pick4(g, r), r + 16 * (r >> 2), 64);  // G_rr
+    if (__any(in_r && !(diag > 0.0))) continue;
+    const double sc = in_r ? 1.0 / sqrt(diag) : 0.0;
+    b *= sc;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) g[c] *= sc * __shfl(sc, (4 * h + c) & 15, 64);
     bool ok = true;
-    for (int p = 0; p < k && ok; ++p) {
-      const int bp = H.rb[first + p];
-      const double dp = D[(size_t)cur * m1 + bp];
-      b[p] = rr - dp;
-      for (int q = 0; q < k; ++q) {
-        const int bq = H.rb[first + q];
-        G[p][q] = rr - dp - D[(size_t)cur * m1 + bq] + D[(size_t)bp * m1 + bq];
+    for (int col = 0; col < k; ++col) {
+      const int hc = 16 * (col >> 2);  // lanes that hold the column
+      const double gc = __shfl(pick4(g, col), r + hc, 64);
+      // the largest |G_rc|, r >= col, the first of equal ones
+      double best = (r >= col && in_r) ? fabs(gc) : -1.0;
+      int piv = r;
+      for (int off = 8; off > 0; off >>= 1) {
+        const double ob = __shfl_xor(best, off, 64);
+        const int op = __shfl_xor(piv, off, 64);
+        if (ob > best || (ob == best && op < piv)) {
+          best = ob;
+          piv = op;
+        }
       }
-      ok = G[p][p] > 0.0;
-      if (ok) sc[p] = 1.0 / sqrt(G[p][p]);
-    }
-    if (!ok) continue;
-    for (int p = 0; p < k; ++p) {
-      b[p] *= sc[p];
-      for (int q = 0; q < k; ++q) G[p][q] *= sc[p] * sc[q];
-    }
-    for (int col = 0; col < k && ok; ++col) {
-      int piv = col;
-      for (int r = col + 1; r < k; ++r)
-        if (fabs(G[r][col]) > fabs(G[piv][col])) piv = r;
-      if (fabs(G[piv][col]) < 1e-12) {
+      // (a value that is no number loses every comparison: the first row stays)
+      if (best < 1.0e-12) {
         ok = false;
         break;
       }
-      if (piv != col) {
-        for (int q = 0; q < k; ++q) {
-          const double tq = G[piv][q];
-          G[piv][q] = G[col][q];
-          G[col][q] = tq;
-        }
-        const double tb = b[piv];
-        b[piv] = b[col];
-        b[col] = tb;
+      const int src = (r == col ? piv : (r == piv ? col : r)) + 16 * h;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) g[c] = __shfl(g[c], src, 64);
+      b = __shfl(b, src, 64);
+      const double gs = __shfl(pick4(g, col), r + hc, 64);
+      const double pv = __shfl(gs, col, 64);
+      const double f = r > col ? gs / pv : 0.0;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const double top = __shfl(g[c], col + 16 * h, 64);
+        if (4 * h + c >= col) g[c] -= f * top;
       }
-      for (int r = col + 1; r < k; ++r) {
-        const double f = G[r][col] / G[col][col];
-        for (int q = col; q < k; ++q) G[r][q] -= f * G[col][q];
-        b[r] -= f * b[col];
-      }
+      const double bt = __shfl(b, col, 64);
+      b -= f * bt;
     }
     if (!ok) continue;
-    for (int r = k - 1; r >= 0; --r) {
-      double a = b[r];
-      for (int q = r + 1; q < k; ++q) a -= G[r][q] * x[q];
-      x[r] = a / G[r][r];
+    double x = 0.0;
+    for (int q = k - 1; q >= 0; --q) {  // back substitution, a column at a time
+      const double gq = __shfl(pick4(g, q), r + 16 * (q >> 2), 64);
+      const double xq = __shfl(b / gq, q, 64);
+      if (r == q) x = xq;
+      if (r < q) b -= gq * xq;
     }
-    for (int p = 0; p < k; ++p) xcoef[first + p] = x[p] * sc[p];
-    return;
+    // entry first + p has row p
+    const double xs = x * sc;
+    th = __shfl(xs, (r - first) & 15, 64);
+    if (r < first) th = 0.0;
+    break;
   }
+  if (lane < nh) xcoef[lane] = th;
 }
 
 // ---------------------------------------------------------------------------
@@ -624,12 +704,23 @@ hipError_t run_reduce_cols(const double *in, size_t nrow, int width, int nsets, 
   return hipGetLastError();
 }
 
-hipError_t run_step_finish(const double *sums, const double *rho, int natv, size_t N,
-                           double tol, int mixing, double mp, int binary, double *scal,
-                           double *rms_hist, int *done, hipStream_t st, const GroupPtrs *grp,
-                           int ngrp) {
-  hipLaunchKernelGGL(k_step_finish, dim3(1, 1, grp ? ngrp : 1), dim3(64), 0, st, sums, rho, natv,
-                     N, tol, mixing, mp, binary, scal, rms_hist, done, grp);
+// threads of the step's end: one row of sums per site needs few
+static int end_threads(bool reduced) { return reduced ? 256 : kEndThreads; }
+
+hipError_t run_step_finish(const double *partial, size_t nrow, double *sums, const double *rho,
+                           int natv, size_t N, double tol, int mixing, double mp, int binary,
+                           double *scal, double *rms_hist, int *done, hipStream_t st,
+                           const GroupPtrs *grp, int ngrp) {
+  const int cols = 6 * natv;
+  const bool reduce = nrow * cols > kOneGroupSums;
+  if (cols > kEndThreads) return hipErrorInvalidValue;
+  if (reduce) {
+    const hipError_t e = run_reduce_cols(partial, nrow, 6, natv, sums, done, st, grp, ngrp);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL(k_step_finish, dim3(1, 1, grp ? ngrp : 1), dim3(end_threads(reduce)), 0, st,
+                     reduce ? sums : partial, reduce ? (size_t)1 : nrow, rho, natv, N, tol, mixing,
+                     mp, binary, scal, rms_hist, done, grp, (int)reduce);
   return hipGetLastError();
 }
 
@@ -674,17 +765,24 @@ hipError_t run_andm_update(Re *tnew, const Re *t, const Re *R, const HistUpdateT
   return hipGetLastError();
 }
 
-hipError_t run_andm_finish(const double *sums, const double *rho, int natv, size_t N, double tol,
-                           int width, double *D, int m1, int cur, const int *rb, int nh,
-                           int mixing, double *xcoef, double *scal, double *rms_hist, int *done,
-                           hipStream_t st) {
-  if (nh < 0 || nh > RISM_MAX_HIST || m1 > RISM_MAX_HIST + 1 || width < 1 + nh)
+hipError_t run_andm_finish(const double *partial, size_t nrow, double *sums, const double *rho,
+                           int natv, size_t N, double tol, int width, double *D, int m1, int cur,
+                           const int *rb, int nh, int mixing, double *xcoef, double *scal,
+                           double *rms_hist, int *done, hipStream_t st) {
+  if (nh < 0 || nh > RISM_MAX_HIST || m1 > RISM_MAX_HIST + 1 || width != 1 + RISM_MAX_HIST ||
+      natv * width > kEndThreads)
     return hipErrorInvalidValue;
   AndmHist H{};
   H.nh = nh;
   for (int p = 0; p < nh; ++p) H.rb[p] = rb[p];
-  hipLaunchKernelGGL(k_andm_finish, dim3(1), dim3(64), 0, st, sums, rho, natv, N, tol, width, D,
-                     m1, cur, H, mixing, xcoef, scal, rms_hist, done);
+  const bool reduce = nrow * natv * width > kOneGroupSums;
+  if (reduce) {
+    const hipError_t e = run_reduce_cols(partial, nrow, width, natv, sums, done, st);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL(k_andm_finish, dim3(1), dim3(end_threads(reduce)), 0, st,
+                     reduce ? sums : partial, reduce ? (size_t)1 : nrow, rho, natv, N, tol, width,
+                     D, m1, cur, H, mixing, xcoef, scal, rms_hist, done);
   return hipGetLastError();
 }
 
