@@ -99,7 +99,7 @@ struct TablesT {
 // before it hands over to FP64).
 template <class Re>
 struct Level {
-  Re *u = nullptr, *fr = nullptr, *T[2] = {}, *Pslot[2] = {}, *R[3] = {};
+  Re *u = nullptr, *fr = nullptr, *T[2] = {}, *Pslot[3] = {}, *R[3] = {};
   cx<Re> *fk = nullptr, *spec = nullptr;
   std::vector<Re *> Rb, Pb;  // Anderson(m) residuals and mixed iterates
   Re *Rlast = nullptr;       // residual written by the last step at this level
@@ -176,8 +176,11 @@ struct rism_ctx {
   int count = 0, binary = 0;
   double lastx[2] = {0, 0}, lasts[2] = {0, 0};
   // t ping-pongs between T[0] and T[1]; slot p holds P_p = T_p + m R_p in
-  // Pslot[p] and R_p in R[iR_slot[p]] (rotated by pointer)
+  // Pslot[iR_slot[p]] and R_p in R[iR_slot[p]] (rotated by pointer; without
+  // memory for Pslot[2], P_p in Pslot[p]).  The residual pass writes t + m R to
+  // Pslot[iR_cur]; q_ok: it did for the t and R at hand.
   int iT_cur = 0, iR_cur = 0, iR_slot[2] = {1, 2};
+  bool q_ok = false;
   int iT_last = 0;
   int last_prec = 0;  // level of the last rism_calculate
   bool fresh = false;  // no rism_anderson since that rism_calculate
@@ -241,6 +244,14 @@ struct rism_ctx {
     allocs.push_back(q);
     *p = (Tp *)q;
     return RISM_OK;
+  }
+  void release(void *p) {
+    for (size_t i = 0; i < allocs.size(); ++i)
+      if (allocs[i] == p) {
+        (void)hipFree(p);
+        allocs.erase(allocs.begin() + i);
+        return;
+      }
   }
   ~rism_ctx() {
     if (gexec) (void)hipGraphExecDestroy(gexec);
@@ -319,6 +330,7 @@ void fill_params(rism_ctx *c) {
   P.dr[1] = c->box[1] / c->ny;
   P.dr[2] = c->box[2] / c->nz;
   for (int d = 0; d < 3; ++d) P.kfac[d] = 2.0 * M_PI / c->box[d];
+  P.mix = c->opts.an2_m;
   for (int v = 0; v < RISM_MAX_SITES; ++v) P.qv[v] = v < c->natv ? c->qv[v] : 0.0;
 }
 
@@ -537,6 +549,12 @@ struct KTime {
   }
 };
 
+// P of AN2 slot p
+template <class Re>
+Re *slot_iterate(const rism_ctx *c, const Level<Re> &L, int p) {
+  return L.Pslot[2] ? L.Pslot[c->iR_slot[p]] : L.Pslot[p];
+}
+
 // One Anderson(m) step: the first an2_count steps are the reference's
 // Picard steps t' = t + R (anderson.cu:54-60); after that
 //   t' = Q + sum_p th_p (P_p - Q),  Q = t + beta R,  beta = an2_m.
@@ -596,14 +614,20 @@ int an2_step(rism_ctx *c) {
   const int oldR = c->iR_slot[b];
   const int *done = c->async ? c->dflag : nullptr;
   Re *t = L.T[c->iT_cur], *R = L.R[c->iR_cur], *tnew = L.T[1 - c->iT_cur];
+  // the iterate that becomes the new slot's: written by the residual pass, or
+  // by the update
+  const bool have = L.Pslot[2] && c->q_ok;
+  Re *Q = L.Pslot[2] ? L.Pslot[c->iR_cur] : L.Pslot[b];
+  Re *P0 = slot_iterate(c, L, 0), *P1 = slot_iterate(c, L, 1);
+  KTime kt(c, RISM_K_AN2);
   if (c->count > 0) {  // anderson.cu:54-60
     --c->count;
-    KTime kt(c, RISM_K_AN2);
-    HIPCHECK(rism::run_an2_picard(tnew, t, R, L.Pslot[b], c->opts.an2_m, nn, done, c->st));
-  } else {  // anderson.cu:61-72
-    KTime kt(c, RISM_K_AN2);
-    HIPCHECK(rism::run_an2_update(tnew, t, R, L.Pslot[0], L.Pslot[1], L.Pslot[b], c->scal,
-                                  c->opts.an2_m, nn, done, c->st));
+    HIPCHECK(rism::run_an2_picard(tnew, t, R, have ? (Re *)nullptr : Q, c->opts.an2_m, nn, done,
+                                  c->st));
+  } else if (have) {  // anderson.cu:61-72
+    HIPCHECK(rism::run_an2_mix(tnew, Q, P0, P1, c->scal, nn, done, c->st));
+  } else {
+    HIPCHECK(rism::run_an2_update(tnew, t, R, P0, P1, Q, c->scal, c->opts.an2_m, nn, done, c->st));
   }
   // slot[b] <- (t, R): P_b was rewritten by the kernel, R_b by pointer
   c->iR_slot[b] = c->iR_cur;
@@ -655,8 +679,9 @@ int calc_step(rism_ctx *c, double *rms, bool lin = false, double tol = -1.0) {
                                    L.tb.zpre, L.tb.zpost, c->st));
     } else {
       const int use_hist = (c->count == 0);
-      HIPCHECK(rism::run_zinv(P, L.spec, t, L.u, Rout, L.R[c->iR_slot[0]], L.R[c->iR_slot[1]],
-                              r0, c->partial, L.tb.twz, L.tb.zpre, L.tb.zpost, use_hist, c->st));
+      HIPCHECK(rism::run_zinv(P, L.spec, t, L.u, Rout,
+                              (L.Pslot[2] && !lin) ? L.Pslot[c->iR_cur] : (Re *)nullptr,
+                              L.R[c->iR_slot[0]], L.R[c->iR_slot[1]], r0, c->partial, L.tb.twz, L.tb.zpre, L.tb.zpost, use_hist, c->st));
     }
   }
   const size_t nb = rism::zinv_num_blocks<Re>(P, andm ? 1 : 0) / c->natv;
@@ -678,6 +703,7 @@ int calc_step(rism_ctx *c, double *rms, bool lin = false, double tol = -1.0) {
     }
   }
   c->iT_last = c->iT_cur;
+  c->q_ok = !lin;
   L.Rlast = Rout;
   c->last_prec = c->prec;
   c->fresh = true;
@@ -713,7 +739,7 @@ int convert_state(rism_ctx *c) {
   int rc;
   for (int i = 0; i < 2; ++i)
     if ((rc = cv(A.T[i], B.T[i]))) return rc;
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < 3; ++i)
     if ((rc = cv(A.Pslot[i], B.Pslot[i]))) return rc;
   for (int i = 0; i < 3; ++i)
     if ((rc = cv(A.R[i], B.R[i]))) return rc;
@@ -728,6 +754,7 @@ int convert_state(rism_ctx *c) {
     if (A.Rlast && A.Rlast == A.Rb[i]) B.Rlast = B.Rb[i];
   HIPCHECK(hipStreamSynchronize(c->st));
   c->last_prec = c->prec = (sizeof(To) == sizeof(double)) ? 0 : 1;
+  c->q_ok = false;
   return RISM_OK;
 }
 
@@ -758,7 +785,7 @@ AccelFields<Re> accel_fields(rism_ctx *c) {
     a.cur = L.Rb[c->cur_rb];
   } else {
     for (int i = 0; i < 2; ++i) {
-      a.iter.push_back(L.Pslot[i]);
+      a.iter.push_back(slot_iterate(c, L, i));
       a.resid.push_back(L.R[c->iR_slot[i]]);
     }
     a.cur = L.R[c->iR_cur];
@@ -783,6 +810,7 @@ int rebase_down(rism_ctx *c, int k0) {
     HIPCHECK(rism::run_convert((const double *)D.resid[i], F.resid[i], nn, c->st));
   HIPCHECK(hipMemsetAsync(c->f.T[k0], 0, sizeof(float) * nn, c->st));
   c->prec = 1;
+  c->q_ok = false;
   return RISM_OK;
 }
 
@@ -1132,7 +1160,7 @@ bool groupable(const rism_ctx *a, const rism_ctx *b) {
          a->solv_hash == b->solv_hash && p.clos == q.clos && p.shell == q.shell &&
          a->opts.an2_count == b->opts.an2_count && a->opts.an2_count <= 32 &&
          a->opts.an2_m == b->opts.an2_m &&
-         a->opts.an2_mp == b->opts.an2_mp && p.var_zf[0] == q.var_zf[0] &&
+         a->opts.an2_mp == b->opts.an2_mp && !a->d.Pslot[2] == !b->d.Pslot[2] && p.var_zf[0] == q.var_zf[0] &&
          p.var_zi[0] == q.var_zi[0] && p.var_y[0] == q.var_y[0] && a->prec == 0 &&
          b->prec == 0 && group_idx(a) == group_idx(b);
 }
@@ -1200,9 +1228,11 @@ int group_tables(GroupRun &g) {
       e.rms_hist = c->rms_hist;
       e.done = c->dflag;
       e.tnew = L.T[1 - ix.iT];
-      e.P0 = L.Pslot[0];
-      e.P1 = L.Pslot[1];
-      e.Pb = L.Pslot[ix.b];
+      const bool q = L.Pslot[2] != nullptr;
+      e.Q = q ? L.Pslot[ix.iR] : nullptr;
+      e.P0 = L.Pslot[q ? ix.s0 : 0];
+      e.P1 = L.Pslot[q ? ix.s1 : 1];
+      e.Pb = q ? nullptr : L.Pslot[ix.b];
       h.push_back(e);
     }
     ix = group_next(ix);
@@ -1236,7 +1266,9 @@ int group_step(GroupRun &g) {
   HIPCHECK(rism::run_y(P, L.spec, -1, L.tb.twy, L.tb.prey, st));
   HIPCHECK(rism::run_xoz(P, L.spec, L.fk, L.tb.twx, L.tb.prex, c->knots, c->coef, L.chitab, st));
   HIPCHECK(rism::run_y(P, L.spec, +1, L.tb.twy, L.tb.prey, st));
-  HIPCHECK(rism::run_zinv(P, L.spec, L.T[ix.iT], L.u, L.R[ix.iR], L.R[ix.s0], L.R[ix.s1],
+  // (in a group the Q, P and slot pointers come from the table)
+  HIPCHECK(rism::run_zinv(P, L.spec, L.T[ix.iT], L.u, L.R[ix.iR], (double *)nullptr, L.R[ix.s0],
+                          L.R[ix.s1],
                           (const double *)nullptr, c->partial, L.tb.twz, L.tb.zpre, L.tb.zpost,
                           ix.count == 0, st));
   const size_t nb = rism::zinv_num_blocks<double>(P, 0) / c->natv;
@@ -1247,6 +1279,9 @@ int group_step(GroupRun &g) {
   if (ix.count > 0) {
     HIPCHECK(rism::run_an2_picard(L.T[1 - ix.iT], L.T[ix.iT], L.R[ix.iR], L.Pslot[ix.b],
                                   c->opts.an2_m, nn, (const int *)nullptr, st, tab, P.ngrp));
+  } else if (L.Pslot[2]) {
+    HIPCHECK(rism::run_an2_mix(L.T[1 - ix.iT], L.Pslot[ix.iR], L.Pslot[ix.s0], L.Pslot[ix.s1],
+                               c->scal, nn, (const int *)nullptr, st, tab, P.ngrp));
   } else {
     HIPCHECK(rism::run_an2_update(L.T[1 - ix.iT], L.T[ix.iT], L.R[ix.iR], L.Pslot[0],
                                   L.Pslot[1], L.Pslot[ix.b], c->scal, c->opts.an2_m, nn,
@@ -1363,10 +1398,10 @@ int setup_enqueue(rism_ctx *c) {
   // history slots start at zero (the reference leaves them uninitialised)
   if (c->opts.anderson_m == 0) {
     for (int i = 0; i < 2; ++i) {
-      HIPCHECK(hipMemsetAsync(c->d.Pslot[i], 0, sizeof(double) * nn, c->st));
+      HIPCHECK(hipMemsetAsync(slot_iterate(c, c->d, i), 0, sizeof(double) * nn, c->st));
       HIPCHECK(hipMemsetAsync(c->d.R[c->iR_slot[i]], 0, sizeof(double) * nn, c->st));
       if (c->opts.precision == 1) {
-        HIPCHECK(hipMemsetAsync(c->f.Pslot[i], 0, sizeof(float) * nn, c->st));
+        HIPCHECK(hipMemsetAsync(slot_iterate(c, c->f, i), 0, sizeof(float) * nn, c->st));
         HIPCHECK(hipMemsetAsync(c->f.R[c->iR_slot[i]], 0, sizeof(float) * nn, c->st));
       }
     }
@@ -1483,7 +1518,8 @@ int tune_launch(rism_ctx *c, int pass) {
                               c->st));
       break;
     case rism::TP_ZINV:
-      HIPCHECK(rism::run_zinv(P, L.spec, L.T[0], L.u, L.R[0], L.R[1], L.R[2], (const Re *)nullptr,
+      HIPCHECK(rism::run_zinv(P, L.spec, L.T[0], L.u, L.R[0], L.Pslot[2], L.R[1], L.R[2],
+                              (const Re *)nullptr,
                               c->partial, L.tb.twz, L.tb.zpre, L.tb.zpost, 1, c->st));
       break;
     default:
@@ -1750,6 +1786,12 @@ rism_ctx *rism_create(const rism_grid *grid, const rism_solvent *solvent,
       hipHostMalloc((void **)&c->hflag, 3 * sizeof(int)) != hipSuccess)
     return fail(rism::set_error(RISM_ERR_NOMEM, "hipHostMalloc failed"));
   if ((rc = make_chi_octant(c))) return fail(rc);
+  // the third AN2 iterate; without memory for it the update forms it itself
+  if (c->opts.anderson_m == 0 && !c->alloc(&c->d.Pslot[2], nn) && c->opts.precision == 1 &&
+      c->alloc(&c->f.Pslot[2], nn)) {
+    c->release(c->d.Pslot[2]);
+    c->d.Pslot[2] = nullptr;
+  }
   if (tune::enabled() || tune::forced(0) >= 0) {
     if ((rc = tune_level<double>(c))) return fail(rc);
     if (c->opts.precision == 1 && (rc = tune_level<float>(c))) return fail(rc);
@@ -2000,6 +2042,7 @@ int rism_set_field(rism_ctx *c, int which, int site, const double *host) {
   if (site < 0 || site >= c->natv) return rism::set_error(RISM_ERR_ARG, "site out of range");
   const size_t off = (size_t)site * c->N;
   if (which == RISM_FIELD_T) {
+    c->q_ok = false;
     if (c->prec == 1) {
       // the FP64 copy is kept too: a mixed solve whose FP32 phase overflows
       // restarts in FP64 from it
@@ -2462,7 +2505,8 @@ int rism_k_fft_c2r(int nx, int ny, int nz, const double box[3], const double *in
   HIPCHECK(rism::run_xoz(P, spec, spec, c->d.tb.twx, c->d.tb.prex, nullptr, nullptr,
                          (const double *)nullptr, c->st));
   HIPCHECK(rism::run_y(P, spec, +1, c->d.tb.twy, c->d.tb.prey, c->st));
-  HIPCHECK(rism::run_zinv(P, spec, h, h, h, h, h, (const double *)nullptr, partial, c->d.tb.twz,
+  HIPCHECK(rism::run_zinv(P, spec, h, h, h, (double *)nullptr, h, h, (const double *)nullptr,
+                          partial, c->d.tb.twz,
                           c->d.tb.zpre, c->d.tb.zpost, 0, c->st));
   HIPCHECK(hipMemcpyAsync(out, h, sizeof(double) * c->N, hipMemcpyDeviceToHost, c->st));
   HIPCHECK(hipStreamSynchronize(c->st));

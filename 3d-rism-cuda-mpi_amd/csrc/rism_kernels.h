@@ -34,6 +34,7 @@ struct GroupPtrs {
   const void *R0, *R1;
   double *partial, *sums, *scal, *rms_hist;
   int *done;
+  void *Q;     // residual pass: t + m R, or null
   void *tnew;  // AN2 update
   const void *P0, *P1;
   void *Pb;
@@ -46,6 +47,7 @@ struct Params {
   int mode;          // 0 solver step; 1 plain forward transform; 2 plain inverse;
                      // 3 difference-form step (correction sweep of the mixed solve)
   int shell;         // chi source: RISM_CHI_SPLINE, _SHELL or _OCTANT
+  double mix;        // AN2 mixing coefficient m (the residual pass's Q = t + m R)
   double dv;         // volume element (forward scale)
   double inv_scale;  // 1 / (dv nx ny (nz/2)): inverse scale of the three passes
   double dr[3];      // grid spacing
@@ -115,9 +117,11 @@ hipError_t run_chi_octant(const double *knots, const double *coef, const Params 
 // AN2 partial sums (6 per workgroup) of the residual pass
 // P.mode 3 (difference form): t = correction d, u = exponent a = -u + t0 at
 // the base point, r0 = the full residual at t0; R = r0 + h - (g(a+d) - g(a)).
+// Q (may be null): t + m R of the step, the mixed iterate the update starts
+// from; not written in mode 3
 template <class Re>
 hipError_t run_zinv(const Params &P, const cx<Re> *spec, const Re *t, const Re *u, Re *R,
-                    const Re *R0, const Re *R1, const Re *r0, double *partial,
+                    Re *Q, const Re *R0, const Re *R1, const Re *r0, double *partial,
                     const cx<Re> *twM, const cx<Re> *zpre, const cx<Re> *zpost, int use_hist,
                     hipStream_t st);
 // Anderson(m) variant: partial sums R.R and R.R_p for the nh history vectors
@@ -162,7 +166,13 @@ template <class Re>
 hipError_t run_an2_picard(Re *tnew, const Re *t, const Re *R, Re *Pb, double m, size_t n,
                           const int *done, hipStream_t st, const GroupPtrs *grp = nullptr,
                           int ngrp = 0);
-// s1, s2 from scal[3], scal[4] (run_step_finish)
+// t' = Q + s1 (P0 - Q) + s2 (P1 - Q), s1, s2 from scal[3], scal[4]
+template <class Re>
+hipError_t run_an2_mix(Re *tnew, const Re *Q, const Re *P0, const Re *P1, const double *scal,
+                       size_t n, const int *done, hipStream_t st, const GroupPtrs *grp = nullptr,
+                       int ngrp = 0);
+// the same from t and R, writing Q to Pb, where the residual pass did not
+// write it.  s1, s2 from scal[3], scal[4] (run_step_finish)
 template <class Re>
 hipError_t run_an2_update(Re *tnew, const Re *t, const Re *R, const Re *P0, const Re *P1, Re *Pb,
                           const double *scal, double m, size_t n, const int *done,

@@ -51,9 +51,14 @@ __global__ void __launch_bounds__(256)
 //   t' = u + m (v - u).
 // Writing Q = t + m R and P_p = T_p + m R_p this is
 //   t' = Q + s1 (P0 - Q) + s2 (P1 - Q),
-// so each slot stores P_p (for the update) and R_p (for the Gram matrix,
-// kept by pointer rotation): the update reads t, R, P0, P1 and writes t'
-// and the retired slot's P = Q, 6 words per point instead of 7.
+// so each slot stores P_p (for the update) and R_p (for the Gram matrix), kept
+// by pointer rotation.
+//
+// The residual pass writes Q into the third of three rotating buffers, which
+// becomes the new slot's P: the update reads Q, P0, P1 and writes t', 4 words
+// per point (k_an2_mix).  Where it did not (no memory for a third buffer, the
+// difference-form steps, a t set by the caller) Q is formed here and written
+// out, 6 words (k_an2_update).
 //
 // Picard warm-up (newdt0): t' = t + R, P_b = t + m R.
 // Both kernels move two consecutive elements per thread as 16-byte accesses
@@ -118,10 +123,36 @@ __global__ void k_an2_picard(V16<Re> *__restrict__ tnew, const V16<Re> *__restri
     b.a[k] = ti.a[k] + mcoef * ri.a[k];
   }
   tnew[i] = a;
-  Pb[i] = b;
+  if (Pb) Pb[i] = b;
 }
 
-// Pb aliases P0 or P1 (the slot being retired); each element is read before
+template <class Re>
+__global__ void k_an2_mix(V16<Re> *__restrict__ tnew, const V16<Re> *__restrict__ Q,
+                          const V16<Re> *__restrict__ P0, const V16<Re> *__restrict__ P1,
+                          const double *__restrict__ scal, size_t nv, const int *done,
+                          const GroupPtrs *grp) {
+  if (grp) {
+    const GroupPtrs &g = grp[blockIdx.z];
+    done = global_ptr<const int>(g.done);
+    tnew = global_ptr<V16<Re>>(g.tnew);
+    Q = global_ptr<const V16<Re>>(g.Q);
+    P0 = global_ptr<const V16<Re>>(g.P0);
+    P1 = global_ptr<const V16<Re>>(g.P1);
+    scal = global_ptr<const double>(g.scal);
+  }
+  if (done && *done) return;
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nv) return;
+  const Re s1 = (Re)scal[3], s2 = (Re)scal[4];
+  const V16<Re> q = ld_nt(Q + i), p0 = ld_nt(P0 + i), p1 = ld_nt(P1 + i);
+  V16<Re> a;
+#pragma unroll
+  for (int k = 0; k < V16<Re>::K; ++k)
+    a.a[k] = q.a[k] + s1 * (p0.a[k] - q.a[k]) + s2 * (p1.a[k] - q.a[k]);
+  st_nt(tnew + i, a);
+}
+
+// Pb may alias P0 or P1 (the slot being retired); each element is read before
 // it is written by the same thread.
 template <class Re>
 __global__ void k_an2_update(V16<Re> *__restrict__ tnew, const V16<Re> *__restrict__ t,
@@ -754,6 +785,17 @@ hipError_t run_an2_update(Re *tnew, const Re *t, const Re *R, const Re *P0, cons
 }
 
 template <class Re>
+hipError_t run_an2_mix(Re *tnew, const Re *Q, const Re *P0, const Re *P1, const double *scal,
+                       size_t n, const int *done, hipStream_t st, const GroupPtrs *grp, int ngrp) {
+  if (n % V16<Re>::K) return hipErrorInvalidValue;
+  const size_t nv = nvec<Re>(n);
+  hipLaunchKernelGGL(k_an2_mix<Re>, dim3(nblk(nv, 256), 1, grp ? ngrp : 1), dim3(256), 0, st,
+                     (V16<Re> *)tnew, (const V16<Re> *)Q, (const V16<Re> *)P0,
+                     (const V16<Re> *)P1, scal, nv, done, grp);
+  return hipGetLastError();
+}
+
+template <class Re>
 hipError_t run_andm_update(Re *tnew, const Re *t, const Re *R, const HistUpdateT<Re> &H, Re *Pb,
                            const double *xcoef, double beta, size_t n, const int *done,
                            hipStream_t st) {
@@ -795,6 +837,9 @@ hipError_t run_convert(const From *in, To *out, size_t n, hipStream_t st) {
 #define INST(Re)                                                                              \
   template hipError_t run_an2_picard<Re>(Re *, const Re *, const Re *, Re *, double, size_t,  \
                                          const int *, hipStream_t, const GroupPtrs *, int);   \
+  template hipError_t run_an2_mix<Re>(Re *, const Re *, const Re *, const Re *,                \
+                                      const double *, size_t, const int *, hipStream_t,        \
+                                      const GroupPtrs *, int);                                 \
   template hipError_t run_an2_update<Re>(Re *, const Re *, const Re *, const Re *, const Re *, \
                                          Re *, const double *, double, size_t, const int *,   \
                                          hipStream_t, const GroupPtrs *, int);                \

@@ -225,8 +225,9 @@ template <int M, int B, int TZ, int HM, int KIND, class Re, int WPE = zinv_waves
 __global__ void __launch_bounds__(B *TZ)
     __attribute__((amdgpu_waves_per_eu(WPE)))
     k_zinv_resid(const cx<Re> *__restrict__ spec, const Re *__restrict__ t,
-                 const Re *__restrict__ u, Re *__restrict__ R, const Re *__restrict__ R0,
-                 const Re *__restrict__ R1, const Re *__restrict__ r0, HistT<Re> H, Params P,
+                 const Re *__restrict__ u, Re *__restrict__ R, Re *__restrict__ Q,
+                 const Re *__restrict__ R0, const Re *__restrict__ R1,
+                 const Re *__restrict__ r0, HistT<Re> H, Params P,
                  double *__restrict__ partial,
                  const cx<Re> *__restrict__ twM, const cx<Re> *__restrict__ zpre,
                  const cx<Re> *__restrict__ zpost) {
@@ -247,6 +248,7 @@ __global__ void __launch_bounds__(B *TZ)
     t = global_ptr<const Re>(g.t);
     u = global_ptr<const Re>(g.u);
     R = global_ptr<Re>(g.R);
+    Q = global_ptr<Re>(g.Q);
     R0 = global_ptr<const Re>(g.R0);
     R1 = global_ptr<const Re>(g.R1);
     partial = global_ptr<double>(g.partial);
@@ -314,6 +316,16 @@ __global__ void __launch_bounds__(B *TZ)
   const Re *tv = t + (size_t)v * N;
   const Re *uv = u + (size_t)v * N;
   Re *Rv = R + (size_t)v * N;
+  // AN2: the mixed iterate Q = t + m R goes out with R while t is at hand, so
+  // that the update reads Q and the two slots instead of t, R and the slots
+  // and writes t' alone (4 words per point and site instead of 6, against one
+  // more here: 512^3, 4 sites, 5.51 + 4.38 -> 5.86 + 2.81 ms; 256^3 0.64 + 0.53
+  // -> 0.65 + 0.35 ms)
+  // (the difference form leaves it to the update: its FP32 tile spills 27 VGPRs
+  // for it at 256 points)
+  constexpr bool kQ = HM == 0 && (KIND == ZK_STEP || KIND == ZK_PICARD);
+  Re *Qv = (kQ && Q) ? Q + (size_t)v * N : nullptr;
+  const Re mix = (Re)P.mix;
   const Re *R0v = R0 + (size_t)v * N;
   const Re *R1v = R1 + (size_t)v * N;
   const size_t base = (size_t)y * P.nx + (ok ? x : 0);
@@ -337,6 +349,9 @@ __global__ void __launch_bounds__(B *TZ)
     else
       rr = h + (Re)1 - closure_g(clos, ti, ui);
     __builtin_nontemporal_store(rr, &Rv[i]);
+    if constexpr (kQ) {
+      if (Qv) __builtin_nontemporal_store(ti + mix * rr, &Qv[i]);
+    }
     // the sums are FP64 whatever the bulk type
     const double r = (double)rr;
     s[0] += r * r;
@@ -376,12 +391,12 @@ __global__ void __launch_bounds__(B *TZ)
         Re t0, t1, u0, u1, a0, a1, b0, b1, c0, c1;
       };
       const Re *tv, *uv, *R0v, *R1v, *r0v;
-      Re *Rv;
+      Re *Rv, *Qv;
       const C *zpre;
       C zprej;
       int j;
       size_t base, plane;
-      Re scale;
+      Re scale, mix;
       int clos;
       bool ok;
       double s[W];
@@ -418,6 +433,9 @@ __global__ void __launch_bounds__(B *TZ)
         else
           rr = h + (Re)1 - closure_g(clos, ti, ui);
         __builtin_nontemporal_store(rr, &Rv[i]);
+        if constexpr (kQ) {
+          if (Qv) __builtin_nontemporal_store(ti + mix * rr, &Qv[i]);
+        }
         // the sums are FP64 whatever the bulk type
         const double r = (double)rr;
         s[0] += r * r;
@@ -438,8 +456,8 @@ __global__ void __launch_bounds__(B *TZ)
         one(i0, zz.x, a.t0, a.u0, a.a0, a.b0, a.c0);
         one(i0 + plane, zz.y, a.t1, a.u1, a.a1, a.b1, a.c1);
       }
-    } store{tv,   uv,   R0v,  R1v,   r0 ? r0 + voff : nullptr, Rv, zpre, zpre[j], j, base,
-            plane, scale, clos, ok, {}};
+    } store{tv,   uv,    R0v,   R1v, r0 ? r0 + voff : nullptr, Rv, Qv, zpre, zpre[j], j, base,
+            plane, scale, mix, clos, ok, {}};
     fft_column<M, +1, false, true, TZ, MAXRI, (WPE <= 2)>(col, j, twM, load, store);
 #pragma unroll
     for (int k = 0; k < W; ++k) s[k] = store.s[k];
@@ -551,13 +569,13 @@ static void launch_zfwd(const Params &P, const Re *t, const Re *u, const Re *fr,
 }
 template <int M, int HM, int KIND, class Re, int V = 0>
 static void launch_zinv(const Params &P, const cx<Re> *spec, const Re *t, const Re *u, Re *R,
-                        const Re *R0, const Re *R1, const Re *r0, const HistT<Re> &H,
+                        Re *Q, const Re *R0, const Re *R1, const Re *r0, const HistT<Re> &H,
                         double *partial, const cx<Re> *twM, const cx<Re> *zpre,
                         const cx<Re> *zpost, hipStream_t st) {
   using Z = ZiPlan<M, Re, HM, V>;
   hipLaunchKernelGGL((k_zinv_resid<M, Z::B, Z::T, HM, KIND, Re, Z::WPE>),
                      dim3(zgrid(P, Z::B), 1, P.grp ? P.ngrp : 1), dim3(Z::B * Z::T), 0, st, spec,
-                     t, u, R, R0, R1, r0, H, P, partial, twM, zpre, zpost);
+                     t, u, R, Q, R0, R1, r0, H, P, partial, twM, zpre, zpost);
 }
 
 // Lengths with more than one plan: the autotuner's search space (smaller
@@ -616,20 +634,20 @@ hipError_t zfwd_dispatch(const Params &P, const Re *t, const Re *u, const Re *fr
 // AN2 and Picard steps of the residual pass in the tuned plan
 template <int M, int KIND, class Re>
 static void zinv_step_plan(const Params &P, const cx<Re> *spec, const Re *t, const Re *u, Re *R,
-                           const Re *R0, const Re *R1, const Re *r0, const HistT<Re> &H,
+                           Re *Q, const Re *R0, const Re *R1, const Re *r0, const HistT<Re> &H,
                            double *partial, const cx<Re> *twM, const cx<Re> *zpre,
                            const cx<Re> *zpost, hipStream_t st) {
   if constexpr (RISM_TUNED(M) && zi_plan_offered<M, Re, 1>()) {
     if (P.var_zi[sizeof(Re) == 4] == 1)
-      return launch_zinv<M, 0, KIND, Re, 1>(P, spec, t, u, R, R0, R1, r0, H, partial, twM,
+      return launch_zinv<M, 0, KIND, Re, 1>(P, spec, t, u, R, Q, R0, R1, r0, H, partial, twM,
                                             zpre, zpost, st);
   }
-  launch_zinv<M, 0, KIND, Re>(P, spec, t, u, R, R0, R1, r0, H, partial, twM, zpre, zpost, st);
+  launch_zinv<M, 0, KIND, Re>(P, spec, t, u, R, Q, R0, R1, r0, H, partial, twM, zpre, zpost, st);
 }
 
 template <class Re>
 hipError_t zinv_dispatch(const Params &P, const cx<Re> *spec, const Re *t, const Re *u, Re *R,
-                         const Re *R0, const Re *R1, const Re *r0, double *partial,
+                         Re *Q, const Re *R0, const Re *R1, const Re *r0, double *partial,
                          const cx<Re> *twM, const cx<Re> *zpre, const cx<Re> *zpost,
                          int use_hist, hipStream_t st) {
   if (P.mode == 3 && !r0) return hipErrorInvalidValue;
@@ -641,16 +659,16 @@ hipError_t zinv_dispatch(const Params &P, const cx<Re> *spec, const Re *t, const
 #define X(n)                                                                              \
   case n:                                                                                 \
     if (kind == ZK_STEP)                                                                  \
-      zinv_step_plan<n, ZK_STEP, Re>(P, spec, t, u, R, R0, R1, r0, H, partial, twM, zpre, \
+      zinv_step_plan<n, ZK_STEP, Re>(P, spec, t, u, R, Q, R0, R1, r0, H, partial, twM, zpre, \
                                      zpost, st);                                          \
     else if (kind == ZK_PICARD)                                                           \
-      zinv_step_plan<n, ZK_PICARD, Re>(P, spec, t, u, R, R0, R1, r0, H, partial, twM,     \
+      zinv_step_plan<n, ZK_PICARD, Re>(P, spec, t, u, R, Q, R0, R1, r0, H, partial, twM,     \
                                        zpre, zpost, st);                                  \
     else if constexpr (sizeof(Re) == 8)                                                   \
-      launch_zinv<n, 0, ZK_PLAIN>(P, spec, t, u, R, R0, R1, r0, H, partial, twM, zpre,    \
+      launch_zinv<n, 0, ZK_PLAIN>(P, spec, t, u, R, Q, R0, R1, r0, H, partial, twM, zpre,    \
                                   zpost, st);                                             \
     else                                                                                  \
-      launch_zinv<n, 0, ZK_DIFF>(P, spec, t, u, R, R0, R1, r0, H, partial, twM, zpre,     \
+      launch_zinv<n, 0, ZK_DIFF>(P, spec, t, u, R, Q, R0, R1, r0, H, partial, twM, zpre,     \
                                  zpost, st);                                              \
     break;
     RISM_LENGTHS(X)
@@ -677,12 +695,12 @@ hipError_t zinv_hist_dispatch(const Params &P, const cx<Re> *spec, const Re *t, 
   case n:                                                                                   \
     if constexpr (sizeof(Re) == 4) {                                                        \
       if (P.mode == 3) {                                                                    \
-        launch_zinv<n, 1, ZK_DIFF>(P, spec, t, u, R, nul, nul, r0, H, partial, twM, zpre,   \
+        launch_zinv<n, 1, ZK_DIFF>(P, spec, t, u, R, (Re *)nullptr, nul, nul, r0, H, partial, twM, zpre,   \
                                    zpost, st);                                              \
         break;                                                                              \
       }                                                                                     \
     }                                                                                       \
-    launch_zinv<n, 1, ZK_STEP>(P, spec, t, u, R, nul, nul, r0, H, partial, twM, zpre, zpost, \
+    launch_zinv<n, 1, ZK_STEP>(P, spec, t, u, R, (Re *)nullptr, nul, nul, r0, H, partial, twM, zpre, zpost, \
                                st);                                                         \
     break;
     RISM_LENGTHS(X)
@@ -732,10 +750,10 @@ hipError_t run_zfwd(const Params &P, const Re *t, const Re *u, const Re *fr, cx<
 }
 template <class Re>
 hipError_t run_zinv(const Params &P, const cx<Re> *spec, const Re *t, const Re *u, Re *R,
-                    const Re *R0, const Re *R1, const Re *r0, double *partial,
+                    Re *Q, const Re *R0, const Re *R1, const Re *r0, double *partial,
                     const cx<Re> *twM, const cx<Re> *zpre, const cx<Re> *zpost, int use_hist,
                     hipStream_t st) {
-  return zinv_dispatch<Re>(P, spec, t, u, R, R0, R1, r0, partial, twM, zpre, zpost, use_hist,
+  return zinv_dispatch<Re>(P, spec, t, u, R, Q, R0, R1, r0, partial, twM, zpre, zpost, use_hist,
                            st);
 }
 template <class Re>
@@ -751,7 +769,7 @@ hipError_t run_zinv_hist(const Params &P, const cx<Re> *spec, const Re *t, const
                                    cx<Re> *, const cx<Re> *, const cx<Re> *, const cx<Re> *,  \
                                    hipStream_t);                                              \
   template hipError_t run_zinv<Re>(const Params &, const cx<Re> *, const Re *, const Re *,    \
-                                   Re *, const Re *, const Re *, const Re *, double *,        \
+                                   Re *, Re *, const Re *, const Re *, const Re *, double *,        \
                                    const cx<Re> *, const cx<Re> *, const cx<Re> *, int,       \
                                    hipStream_t);                                              \
   template hipError_t run_zinv_hist<Re>(const Params &, const cx<Re> *, const Re *,           \

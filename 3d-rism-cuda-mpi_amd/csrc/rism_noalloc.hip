@@ -115,7 +115,8 @@ extern "C" int rism_k_fft_noalloc(int dir, int nx, int ny, int nz, const double 
     NA_CHECK(rism::run_apply_phase(sp, P, 1, st));
     NA_CHECK(rism::run_xoz(P, sp, sp, twx, prex, nullptr, nullptr, (const double *)nullptr, st));
     NA_CHECK(rism::run_y(P, sp, +1, twy, prey, st));
-    NA_CHECK(rism::run_zinv(P, sp, real, real, real, real, real, (const double *)nullptr,
+    NA_CHECK(rism::run_zinv(P, sp, real, real, real, (double *)nullptr, real, real,
+                            (const double *)nullptr,
                             partial, twz, zpre, zpost, 0, st));
   }
   return RISM_OK;
