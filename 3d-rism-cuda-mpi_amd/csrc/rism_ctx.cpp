@@ -2323,21 +2323,27 @@ int rism_analysis(rism_ctx *c, int kind, double *out) {
   if (nu == 0) return RISM_OK;
   // cal_LJ.cu:33-44: sigma_uv (lambda-scaled for -l), eps_uv = sqrt(eps_u eps_v)
   const double lam1 = (c->opts.ad_switch == 1) ? c->opts.lambda : 1.0;
-  std::vector<double> adata((size_t)nu * (4 + 2 * nv));
-  for (int a = 0; a < nu; ++a) {
-    double *p = adata.data() + (size_t)a * (4 + 2 * nv);
-    p[0] = c->uxyz[3 * a];
-    p[1] = c->uxyz[3 * a + 1];
-    p[2] = c->uxyz[3 * a + 2];
-    p[3] = c->uq[a];
-    for (int v = 0; v < nv; ++v) {
-      p[4 + v] = (c->usig[a] + c->sigv[v]) * 0.5 * lam1;
-      p[4 + nv + v] = std::sqrt(c->ueps[a] * c->epsv[v]);
-    }
-  }
+  const double cc = kHartree * kBohr * kAvogadro;  // cal_grad.cu:47
   const int k = kind == RISM_ANALYSIS_GRAD ? 0
               : kind == RISM_ANALYSIS_EUV  ? 1
               : (c->opts.ad_switch == 1 ? 2 : 3);
+  const int stride = rism::atom_sum_stride(nv);
+  std::vector<double> adata((size_t)nu * stride);
+  for (int a = 0; a < nu; ++a) {
+    double *p = adata.data() + (size_t)a * stride;
+    for (int d = 0; d < 3; ++d) p[d] = c->uxyz[3 * (size_t)a + d];
+    for (int v = 0; v < nv; ++v) {
+      const double sg = (c->usig[a] + c->sigv[v]) * 0.5 * lam1;
+      const double eps = std::sqrt(c->ueps[a] * c->epsv[v]);
+      const double cut = (k == 2 ? sg * c->opts.lambda : sg) * 0.5;
+      const double s2 = sg * sg;
+      double *q = p + 3 + 4 * v;
+      q[0] = cut * cut;
+      q[1] = s2 * s2 * s2;
+      q[2] = k == 1 ? 4.0 * eps : (k == 2 ? 24.0 * eps / c->opts.lambda : 24.0 * eps);
+      q[3] = cc * c->uq[a] * c->qv[v];
+    }
+  }
   const int width = k == 0 ? 3 : (k == 1 ? nv : 1);
   const size_t nslab = (c->N + rism::atom_sum_slab(c->N) - 1) / rism::atom_sum_slab(c->N);
   double *dad = nullptr, *dpart = nullptr, *dout = nullptr;
@@ -2354,12 +2360,11 @@ int rism_analysis(rism_ctx *c, int kind, double *out) {
     return rism::set_error(RISM_ERR_NOMEM, "hipMalloc failed in rism_analysis");
   }
   std::vector<double> sums((size_t)nu * width);
-  const double cc = kHartree * kBohr * kAvogadro;  // cal_grad.cu:47
   hipError_t e = hipMemcpyAsync(dad, adata.data(), sizeof(double) * adata.size(),
                                 hipMemcpyHostToDevice, c->st);
   if (e == hipSuccess)
-    e = rism::run_atom_sums(k, c->d.T[c->iT_last], c->d.u, c->P, dad, nu,
-                            c->opts.lambda, cc, c->rho_dev, dpart, c->st);
+    e = rism::run_atom_sums(k, c->d.T[c->iT_last], c->d.u, c->P, dad, nu, c->rho_dev, dpart,
+                            c->st);
   if (e == hipSuccess)
     e = rism::run_reduce_cols(dpart, nslab, nu * width, 1, dout, nullptr, c->st);
   if (e == hipSuccess)

@@ -213,11 +213,15 @@ hipError_t run_apply_phase(cplx *s, const Params &P, int inverse, hipStream_t st
 // pre(ny), zpre, zpost (the order of a context's host-computed tables)
 hipError_t run_fft_tables(int nx, int ny, int nz, cplx *tw, hipStream_t st);
 // per-atom integrals of g (kind 0 grad, 1 euv, 2 ad1, 3 ad2); adata: per atom
-// x y z q sigma_uv[natv] eps_uv[natv]; partial: [slab][natu][width] with
-// width 3, natv, 1, 1 and atom_sum_slab(N) points per slab
+// atom_sum_stride(natv) values: x y z, then per site the squared cutoff
+// (sigma_uv / 2, times lambda for kind 2), sigma_uv^6, the kind's
+// Lennard-Jones factor (24 eps_uv, 4 eps_uv, 24 eps_uv / lambda) and the
+// Coulomb factor E_h a_0 N_A q_u q_v; partial: [slab][natu][width] with width
+// 3, natv, 1, 1 and atom_sum_slab(N) points per slab
+int atom_sum_stride(int natv);
 size_t atom_sum_slab(size_t N);
 hipError_t run_atom_sums(int kind, const double *t, const double *u, const Params &P,
-                         const double *adata, int natu, double lambda, double cc,
-                         const double *rho, double *partial, hipStream_t st);
+                         const double *adata, int natu, const double *rho, double *partial,
+                         hipStream_t st);
 
 }  // namespace rism

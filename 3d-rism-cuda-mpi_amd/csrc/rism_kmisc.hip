@@ -514,109 +514,127 @@ __global__ void k_convert(const From *__restrict__ in, To *__restrict__ out, siz
 //   kind 2 (ad1):   24 eps s6 (2 s6 - 1) / lambda
 //   kind 3 (ad2):   cc q_u q_v / r
 // with s6 = (sigma_uv^2 / r^2)^3, eps = sqrt(eps_u eps_v) in J/mol, cc =
-// E_h a_0 N_A; kinds 0, 2, 3 weight each site by rho_v.  One thread per atom
-// (atoms in registers), grid points with their g values staged in LDS; each
-// workgroup covers one slab of points and writes its sums per atom.
+// E_h a_0 N_A; kinds 0, 2, 3 weight each site by rho_v.
+// Lanes are grid points and a wave keeps the sums of AT atoms in registers
+// (one thread per atom left most of a workgroup idle for a molecule's few
+// atoms: 80 x 72 x 96, 40 atoms, 2 sites, grad 1112 us and energies 989, now 97
+// and 81).  The
+// four waves of a workgroup take AT atoms each and share g, formed once per
+// point and staged in LDS; 1/r and its powers serve all sites.  FP64 VALU
+// work, about 21 + 9 natv operations a pair.
 // ---------------------------------------------------------------------------
-constexpr int AS_TILE = 256;
+constexpr int AS_TILE = 256;   // points staged at a time
+constexpr int AS_WAVES = 4;
 
-template <int KIND>
-__global__ void __launch_bounds__(256)
+// atoms of a wave: the per-site sums of kind 1 take natv registers each
+template <int KIND, int NVM>
+constexpr int as_atoms() {
+  return (KIND == 1 && NVM > 4) ? 4 : 8;
+}
+// values per atom record: x, y, z, then per site the squared cutoff, sigma^6,
+// the Lennard-Jones factor of the kind and cc q_u q_v
+__host__ __device__ constexpr int as_stride(int natv) { return 3 + 4 * natv; }
+
+template <int KIND, int NVM>
+__global__ void __launch_bounds__(64 * AS_WAVES)
     k_atom_sums(const double *__restrict__ t, const double *__restrict__ u, Params P,
-                const double *__restrict__ adata, int natu, double lambda, double cc,
-                const double *__restrict__ rho, size_t slab, int width,
-                double *__restrict__ partial) {
-  __shared__ double sp[AS_TILE * (3 + RISM_MAX_SITES / 2)];
-  const int nv = P.natv;
-  const int a = blockIdx.x * blockDim.x + threadIdx.x;
-  const bool active = a < natu;
-  // atom record: x y z q, then sigma_uv[nv], eps_uv[nv], q_v folded below
-  const double *ad = adata + (size_t)(active ? a : 0) * (4 + 2 * nv);
-  const double ax = ad[0], ay = ad[1], az = ad[2], aq = ad[3];
-  double acc[KIND == 0 ? 3 : (KIND == 1 ? 8 : 1)];
+                const double *__restrict__ adata, int natu, const double *__restrict__ rho,
+                size_t slab, double *__restrict__ partial) {
+  constexpr int AT = as_atoms<KIND, NVM>();
+  constexpr int W = KIND == 0 ? 3 : (KIND == 1 ? NVM : 1);
+  __shared__ double sg[NVM][AS_TILE];
+  const int nv = P.natv, st = as_stride(nv);
+  const int lane = threadIdx.x & 63;
+  const int a0 = __builtin_amdgcn_readfirstlane((blockIdx.x * AS_WAVES + (threadIdx.x >> 6)) * AT);
+  double acc[AT][W];
 #pragma unroll
-  for (int k = 0; k < (int)(sizeof(acc) / sizeof(double)); ++k) acc[k] = 0.0;
+  for (int a = 0; a < AT; ++a)
+#pragma unroll
+    for (int k = 0; k < W; ++k) acc[a][k] = 0.0;
   const size_t N = (size_t)P.nx * P.ny * P.nz;
   const size_t p0 = (size_t)blockIdx.y * slab;
   const size_t p1 = p0 + slab < N ? p0 + slab : N;
-  double *px = sp, *py = sp + AS_TILE, *pz = sp + 2 * AS_TILE, *pg = sp + 3 * AS_TILE;
   for (size_t q0 = p0; q0 < p1; q0 += AS_TILE) {
     const int nq = (int)((p1 - q0) < (size_t)AS_TILE ? (p1 - q0) : (size_t)AS_TILE);
     __syncthreads();
-    for (int k = threadIdx.x; k < nq; k += blockDim.x) {
-      const size_t i = q0 + k;
-      const int x = (int)(i % P.nx), y = (int)((i / P.nx) % P.ny), z = (int)(i / ((size_t)P.nx * P.ny));
-      px[k] = (double)(x - P.nx / 2) * P.dr[0];
-      py[k] = (double)(y - P.ny / 2) * P.dr[1];
-      pz[k] = (double)(z - P.nz / 2) * P.dr[2];
-    }
-    // g of every site for the tile, AS_TILE doubles per site (in two halves
-    // of the LDS when nv > 4)
-    for (int vh = 0; vh < nv; vh += 4) {
-      const int nvh = nv - vh < 4 ? nv - vh : 4;
-      for (int k = threadIdx.x; k < nq * nvh; k += blockDim.x) {
-        const int w = k / nq, kk = k % nq;
-        const size_t i = (size_t)(vh + w) * N + q0 + kk;
-        pg[w * AS_TILE + kk] = closure_g(P.clos, t[i], u[i]);
-      }
-      __syncthreads();
-      if (active) {
-        for (int w = 0; w < nvh; ++w) {
-          const int v = vh + w;
-          const double sg = ad[4 + v], eps = ad[4 + nv + v];
-          const double cut = (KIND == 2 ? sg * lambda : sg) * 0.5;
-          const double cut2 = cut * cut;
-          const double sg2 = sg * sg;
-          const double qq = cc * aq * P.qv[v];
-          const double wv = (KIND == 1) ? 1.0 : rho[v];
-          double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-          for (int k = 0; k < nq; ++k) {
-            const double dx = px[k] - ax, dy = py[k] - ay, dz = pz[k] - az;
-            const double r2 = dx * dx + dy * dy + dz * dz;
-            if (r2 < cut2) continue;  // r < sigma / 2 (r = 0 included)
-            const double g = pg[w * AS_TILE + k];
-            const double ir = rsq_nr(r2);
-            const double ir2 = ir * ir;
-            const double rs2 = sg2 * ir2, rs6 = rs2 * rs2 * rs2;
-            if (KIND == 0) {
-              const double f = (eps * 24.0 * rs6 * ir2 * (2.0 * rs6 - 1.0) + qq * ir2 * ir) * g;
-              s0 += f * dx;
-              s1 += f * dy;
-              s2 += f * dz;
-            } else if (KIND == 1) {
-              s0 += (eps * 4.0 * rs6 * (rs6 - 1.0) + qq * ir) * g;
-            } else if (KIND == 2) {
-              s0 += eps * 24.0 * rs6 * (2.0 * rs6 - 1.0) / lambda * g;
-            } else {
-              s0 += qq * ir * g;
-            }
-          }
-          if (KIND == 0) {
-            acc[0] += wv * s0;
-            acc[1] += wv * s1;
-            acc[2] += wv * s2;
-          } else if (KIND == 1) {
+    // g of every site, weighted; zero past the slab's end
 #pragma unroll
-            for (int k = 0; k < 8; ++k)
-              if (k == v) acc[k] += s0;
-          } else {
-            acc[0] += wv * s0;
+    for (int v = 0; v < NVM; ++v) {
+      if (v < nv) {
+        const int k = threadIdx.x;
+        double g = 0.0;
+        if (k < nq) {
+          const size_t i = (size_t)v * N + q0 + k;
+          g = closure_g(P.clos, t[i], u[i]);
+          if (KIND != 1) g *= rho[v];
+        }
+        sg[v][k] = g;
+      }
+    }
+    __syncthreads();
+    if (a0 >= natu) continue;
+    for (int k = lane; k < AS_TILE; k += 64) {
+      // past the end: the last point, whose g is zero
+      const size_t i = q0 + (k < nq ? k : nq - 1);
+      const int x = (int)(i % P.nx), y = (int)((i / P.nx) % P.ny),
+                z = (int)(i / ((size_t)P.nx * P.ny));
+      const double px = (double)(x - P.nx / 2) * P.dr[0], py = (double)(y - P.ny / 2) * P.dr[1],
+                   pz = (double)(z - P.nz / 2) * P.dr[2];
+      double g[NVM];
+#pragma unroll
+      for (int v = 0; v < NVM; ++v) g[v] = v < nv ? sg[v][k] : 0.0;
+#pragma unroll
+      for (int a = 0; a < AT; ++a) {
+        // (a spare atom repeats the last one; its sums are not written)
+        const double *ad = adata + (size_t)(a0 + a < natu ? a0 + a : natu - 1) * st;
+        const double dx = px - ad[0], dy = py - ad[1], dz = pz - ad[2];
+        const double r2 = dx * dx + dy * dy + dz * dz;
+        const double ir = rsq_nr(r2);  // NaN at r = 0: inside every cutoff
+        const double ir2 = ir * ir, ir6 = ir2 * ir2 * ir2;
+        double f = 0.0;
+#pragma unroll
+        for (int v = 0; v < NVM; ++v) {
+          if (v < nv) {
+            const double *as = ad + 3 + 4 * v;
+            const double s6 = as[1] * ir6;
+            double e;
+            if (KIND == 0)
+              e = fma(as[2] * ir2 * s6, fma(2.0, s6, -1.0), as[3] * (ir2 * ir));
+            else if (KIND == 1)
+              e = fma(as[2] * s6, s6 - 1.0, as[3] * ir);
+            else if (KIND == 2)
+              e = as[2] * s6 * fma(2.0, s6, -1.0);
+            else
+              e = as[3] * ir;
+            // r < sigma / 2 is left out (r = 0 included)
+            const bool in = r2 >= as[0];
+            if constexpr (KIND == 1)
+              acc[a][v] += in ? e * g[v] : 0.0;
+            else
+              f += in ? e * g[v] : 0.0;
           }
         }
+        if constexpr (KIND == 0) {
+          acc[a][0] = fma(f, dx, acc[a][0]);
+          acc[a][1] = fma(f, dy, acc[a][1]);
+          acc[a][2] = fma(f, dz, acc[a][2]);
+        } else if constexpr (KIND != 1) {
+          acc[a][0] += f;
+        }
       }
-      __syncthreads();
     }
   }
-  if (!active) return;
-  double *out = partial + ((size_t)blockIdx.y * natu + a) * width;
-  if (KIND == 1) {
+  if (a0 >= natu) return;
+  const int width = KIND == 0 ? 3 : (KIND == 1 ? nv : 1);
 #pragma unroll
-    for (int k = 0; k < 8; ++k)
-      if (k < nv) out[k] = acc[k];
-  } else {
+  for (int a = 0; a < AT; ++a)
 #pragma unroll
-    for (int k = 0; k < (int)(sizeof(acc) / sizeof(double)); ++k) out[k] = acc[k];
-  }
+    for (int k = 0; k < W; ++k) {
+      double x = acc[a][k];
+      for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+      if (lane == 0 && a0 + a < natu && k < width)
+        partial[((size_t)blockIdx.y * natu + a0 + a) * width + k] = x;
+    }
 }
 
 // t = q_v fr (initialize_tuv.cu:19-23)
@@ -755,7 +773,6 @@ hipError_t run_step_finish(const double *partial, size_t nrow, double *sums, con
   return hipGetLastError();
 }
 
-
 template <class Re>
 static size_t nvec(size_t n) {
   return n / V16<Re>::K;
@@ -772,6 +789,17 @@ hipError_t run_an2_picard(Re *tnew, const Re *t, const Re *R, Re *Pb, double m, 
 }
 
 template <class Re>
+hipError_t run_an2_mix(Re *tnew, const Re *Q, const Re *P0, const Re *P1, const double *scal,
+                       size_t n, const int *done, hipStream_t st, const GroupPtrs *grp, int ngrp) {
+  if (n % V16<Re>::K) return hipErrorInvalidValue;
+  const size_t nv = nvec<Re>(n);
+  hipLaunchKernelGGL(k_an2_mix<Re>, dim3(nblk(nv, 256), 1, grp ? ngrp : 1), dim3(256), 0, st,
+                     (V16<Re> *)tnew, (const V16<Re> *)Q, (const V16<Re> *)P0,
+                     (const V16<Re> *)P1, scal, nv, done, grp);
+  return hipGetLastError();
+}
+
+template <class Re>
 hipError_t run_an2_update(Re *tnew, const Re *t, const Re *R, const Re *P0, const Re *P1, Re *Pb,
                           const double *scal, double m, size_t n, const int *done,
                           hipStream_t st, const GroupPtrs *grp, int ngrp) {
@@ -781,17 +809,6 @@ hipError_t run_an2_update(Re *tnew, const Re *t, const Re *R, const Re *P0, cons
                      (V16<Re> *)tnew, (const V16<Re> *)t, (const V16<Re> *)R,
                      (const V16<Re> *)P0, (const V16<Re> *)P1, (V16<Re> *)Pb, scal, (Re)m, nv,
                      done, grp);
-  return hipGetLastError();
-}
-
-template <class Re>
-hipError_t run_an2_mix(Re *tnew, const Re *Q, const Re *P0, const Re *P1, const double *scal,
-                       size_t n, const int *done, hipStream_t st, const GroupPtrs *grp, int ngrp) {
-  if (n % V16<Re>::K) return hipErrorInvalidValue;
-  const size_t nv = nvec<Re>(n);
-  hipLaunchKernelGGL(k_an2_mix<Re>, dim3(nblk(nv, 256), 1, grp ? ngrp : 1), dim3(256), 0, st,
-                     (V16<Re> *)tnew, (const V16<Re> *)Q, (const V16<Re> *)P0,
-                     (const V16<Re> *)P1, scal, nv, done, grp);
   return hipGetLastError();
 }
 
@@ -894,36 +911,42 @@ hipError_t run_thermo_partial(const Re *t, const Re *th, const Re *u,
   return hipGetLastError();
 }
 
+int atom_sum_stride(int natv) { return as_stride(natv); }
+
+// points per workgroup: whole tiles, at most 1024 slabs
 size_t atom_sum_slab(size_t N) {
   size_t s = N / 1024;
-  if (s < 4096) s = 4096;
+  if (s < 1024) s = 1024;
   return (s + AS_TILE - 1) / AS_TILE * AS_TILE;
 }
 
+template <int KIND>
+static void launch_atom_sums(const double *t, const double *u, const Params &P,
+                             const double *adata, int natu, const double *rho, double *partial,
+                             hipStream_t st) {
+  const size_t N = (size_t)P.nx * P.ny * P.nz, slab = atom_sum_slab(N);
+  const unsigned ns = (unsigned)((N + slab - 1) / slab);
+  auto go = [&](auto kern, int at) {
+    hipLaunchKernelGGL(kern, dim3(nblk(natu, AS_WAVES * at), ns), dim3(64 * AS_WAVES), 0, st, t, u,
+                       P, adata, natu, rho, slab, partial);
+  };
+  if (P.natv <= 2)
+    go(k_atom_sums<KIND, 2>, as_atoms<KIND, 2>());
+  else if (P.natv <= 4)
+    go(k_atom_sums<KIND, 4>, as_atoms<KIND, 4>());
+  else
+    go(k_atom_sums<KIND, 8>, as_atoms<KIND, 8>());
+}
+
 hipError_t run_atom_sums(int kind, const double *t, const double *u, const Params &P,
-                         const double *adata, int natu, double lambda, double cc,
-                         const double *rho, double *partial, hipStream_t st) {
-  const size_t N = (size_t)P.nx * P.ny * P.nz;
-  const size_t slab = atom_sum_slab(N);
-  const int width = kind == 0 ? 3 : (kind == 1 ? P.natv : 1);
-  dim3 grid((natu + 255) / 256, (unsigned)((N + slab - 1) / slab));
+                         const double *adata, int natu, const double *rho, double *partial,
+                         hipStream_t st) {
+  if (natu < 1 || P.natv > 8) return hipErrorInvalidValue;
   switch (kind) {
-    case 0:
-      hipLaunchKernelGGL(k_atom_sums<0>, grid, dim3(256), 0, st, t, u, P, adata, natu, lambda,
-                         cc, rho, slab, width, partial);
-      break;
-    case 1:
-      hipLaunchKernelGGL(k_atom_sums<1>, grid, dim3(256), 0, st, t, u, P, adata, natu, lambda,
-                         cc, rho, slab, width, partial);
-      break;
-    case 2:
-      hipLaunchKernelGGL(k_atom_sums<2>, grid, dim3(256), 0, st, t, u, P, adata, natu, lambda,
-                         cc, rho, slab, width, partial);
-      break;
-    default:
-      hipLaunchKernelGGL(k_atom_sums<3>, grid, dim3(256), 0, st, t, u, P, adata, natu, lambda,
-                         cc, rho, slab, width, partial);
-      break;
+    case 0: launch_atom_sums<0>(t, u, P, adata, natu, rho, partial, st); break;
+    case 1: launch_atom_sums<1>(t, u, P, adata, natu, rho, partial, st); break;
+    case 2: launch_atom_sums<2>(t, u, P, adata, natu, rho, partial, st); break;
+    default: launch_atom_sums<3>(t, u, P, adata, natu, rho, partial, st); break;
   }
   return hipGetLastError();
 }
