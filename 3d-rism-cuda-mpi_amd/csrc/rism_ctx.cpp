@@ -2482,7 +2482,6 @@ int rism_k_fft_r2c(int nx, int ny, int nz, const double box[3], const double *in
   HIPCHECK(rism::run_y(P, spec, -1, c->d.tb.twy, c->d.tb.prey, c->st));
   HIPCHECK(rism::run_xoz(P, spec, spec, c->d.tb.twx, c->d.tb.prex, nullptr, nullptr,
                          (const double *)nullptr, c->st));
-  HIPCHECK(rism::run_apply_phase(spec, P, 0, c->st));
   HIPCHECK(hipMemcpyAsync(out, spec, sizeof(cplx) * (c->N / 2), hipMemcpyDeviceToHost, c->st));
   HIPCHECK(hipStreamSynchronize(c->st));
   return RISM_OK;
@@ -2506,7 +2505,6 @@ int rism_k_fft_c2r(int nx, int ny, int nz, const double box[3], const double *in
   HIPCHECK(hipMemcpy(spec, in, sizeof(cplx) * (c->N / 2), hipMemcpyHostToDevice));
   rism::Params P = c->P;
   P.mode = 2;
-  HIPCHECK(rism::run_apply_phase(spec, P, 1, c->st));
   HIPCHECK(rism::run_xoz(P, spec, spec, c->d.tb.twx, c->d.tb.prex, nullptr, nullptr,
                          (const double *)nullptr, c->st));
   HIPCHECK(rism::run_y(P, spec, +1, c->d.tb.twy, c->d.tb.prey, c->st));
@@ -2522,7 +2520,7 @@ int rism_k_get_fk(rism_ctx *c, double *out) {
   if (!c || !out) return rism::set_error(RISM_ERR_ARG, "null argument");
   cplx *tmp = c->d.spec;  // borrow the spectrum buffer
   HIPCHECK(hipMemcpyAsync(tmp, c->d.fk, sizeof(cplx) * (c->N / 2), hipMemcpyDeviceToDevice, c->st));
-  HIPCHECK(rism::run_apply_phase(tmp, c->P, 0, c->st));
+  HIPCHECK(rism::run_apply_phase(tmp, c->P, c->st));
   HIPCHECK(hipMemcpyAsync(out, tmp, sizeof(cplx) * (c->N / 2), hipMemcpyDeviceToHost, c->st));
   HIPCHECK(hipStreamSynchronize(c->st));
   return RISM_OK;

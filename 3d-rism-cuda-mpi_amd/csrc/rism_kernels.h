@@ -207,7 +207,7 @@ hipError_t run_fields(const Re *t, const Re *u, const Re *R, const Params &P, si
 template <class Re>
 hipError_t run_thermo_partial(const Re *t, const Re *th, const Re *u, const Re *R,
                               const Params &P, size_t N, double *partial, hipStream_t st);
-hipError_t run_apply_phase(cplx *s, const Params &P, int inverse, hipStream_t st);
+hipError_t run_apply_phase(cplx *s, const Params &P, hipStream_t st);
 // twiddle and phase tables of the axis passes, computed on the device into
 // tw[2 nx + 2 ny + 3 nz/2]: roots(nx), roots(ny), roots(nz/2), pre(nx),
 // pre(ny), zpre, zpost (the order of a context's host-computed tables)

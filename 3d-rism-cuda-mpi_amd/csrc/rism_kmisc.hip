@@ -713,9 +713,9 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// reference-convention spectrum from a raw one (tests): F = phi * D,
-// phi = -i (-1)^(nx/2 + ny/2 + jx + jy + m); scaled by `scale`.
-__global__ void k_apply_phase(cplx *__restrict__ s, Params P, int inverse) {
+// reference-convention spectrum from a raw one (rism_k_get_fk): F = phi * D,
+// phi = -i (-1)^(nx/2 + ny/2 + jx + jy + m)
+__global__ void k_apply_phase(cplx *__restrict__ s, Params P) {
   const size_t M = P.nz / 2;
   const size_t n = M * P.ny * P.nx;
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -723,8 +723,7 @@ __global__ void k_apply_phase(cplx *__restrict__ s, Params P, int inverse) {
   const int jx = (int)(i % P.nx), jy = (int)((i / P.nx) % P.ny), m = (int)(i / ((size_t)P.nx * P.ny));
   const int sg = ((P.nx / 2 + P.ny / 2 + jx + jy + m) & 1) ? -1 : 1;
   const cplx a = s[i];
-  // phi = -i sg : (x, y) -> sg * (y, -x); conj(phi) = i sg : sg * (-y, x)
-  s[i] = inverse ? mk(-sg * a.y, sg * a.x) : mk(sg * a.y, -sg * a.x);
+  s[i] = mk(sg * a.y, -sg * a.x);  // phi = -i sg
 }
 
 // Plain streaming copy of n 16-byte vectors: the reference point for the HBM
@@ -994,9 +993,9 @@ hipError_t run_fft_tables(int nx, int ny, int nz, cplx *tw, hipStream_t st) {
   return hipGetLastError();
 }
 
-hipError_t run_apply_phase(cplx *s, const Params &P, int inverse, hipStream_t st) {
+hipError_t run_apply_phase(cplx *s, const Params &P, hipStream_t st) {
   const size_t n = (size_t)(P.nz / 2) * P.ny * P.nx;
-  hipLaunchKernelGGL(k_apply_phase, dim3(nblk(n, 256)), dim3(256), 0, st, s, P, inverse);
+  hipLaunchKernelGGL(k_apply_phase, dim3(nblk(n, 256)), dim3(256), 0, st, s, P);
   return hipGetLastError();
 }
 

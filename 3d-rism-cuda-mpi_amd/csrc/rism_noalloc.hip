@@ -109,10 +109,8 @@ extern "C" int rism_k_fft_noalloc(int dir, int nx, int ny, int nz, const double 
                             (const double *)real, sp, twz, zpre, zpost, st));
     NA_CHECK(rism::run_y(P, sp, -1, twy, prey, st));
     NA_CHECK(rism::run_xoz(P, sp, sp, twx, prex, nullptr, nullptr, (const double *)nullptr, st));
-    NA_CHECK(rism::run_apply_phase(sp, P, 0, st));
   } else {  // the steps of rism_k_fft_c2r; the spectrum is the workspace
     P.mode = 2;
-    NA_CHECK(rism::run_apply_phase(sp, P, 1, st));
     NA_CHECK(rism::run_xoz(P, sp, sp, twx, prex, nullptr, nullptr, (const double *)nullptr, st));
     NA_CHECK(rism::run_y(P, sp, +1, twy, prey, st));
     NA_CHECK(rism::run_zinv(P, sp, real, real, real, (double *)nullptr, real, real,
