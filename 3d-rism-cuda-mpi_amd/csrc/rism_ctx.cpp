@@ -654,18 +654,28 @@ int calc_step(rism_ctx *c, double *rms, bool lin = false, double tol = -1.0) {
     KTime kt(c, RISM_K_ZFWD);
     HIPCHECK(rism::run_zfwd(P, t, L.u, L.fr, L.spec, L.tb.twz, L.tb.zpre, L.tb.zpost, c->st));
   }
-  {
-    KTime kt(c, RISM_K_YFWD);
-    HIPCHECK(rism::run_y(P, L.spec, -1, L.tb.twy, L.tb.prey, c->st));
+  bool plane = false;
+  if constexpr (std::is_same<Re, double>::value) {
+    if ((plane = rism::plane_offered(P))) {
+      KTime kt(c, RISM_K_XOZ);
+      HIPCHECK(rism::run_plane(P, L.spec, L.fk, L.tb.twx, L.tb.prex, L.tb.twy, L.tb.prey,
+                               L.chitab, c->st));
+    }
   }
-  {
-    KTime kt(c, RISM_K_XOZ);
-    HIPCHECK(rism::run_xoz(P, L.spec, L.fk, L.tb.twx, L.tb.prex, c->knots, c->coef, L.chitab,
-                           c->st));
-  }
-  {
-    KTime kt(c, RISM_K_YINV);
-    HIPCHECK(rism::run_y(P, L.spec, +1, L.tb.twy, L.tb.prey, c->st));
+  if (!plane) {
+    {
+      KTime kt(c, RISM_K_YFWD);
+      HIPCHECK(rism::run_y(P, L.spec, -1, L.tb.twy, L.tb.prey, c->st));
+    }
+    {
+      KTime kt(c, RISM_K_XOZ);
+      HIPCHECK(rism::run_xoz(P, L.spec, L.fk, L.tb.twx, L.tb.prex, c->knots, c->coef, L.chitab,
+                             c->st));
+    }
+    {
+      KTime kt(c, RISM_K_YINV);
+      HIPCHECK(rism::run_y(P, L.spec, +1, L.tb.twy, L.tb.prey, c->st));
+    }
   }
   const bool andm = c->opts.anderson_m > 0;
   Re *Rout = andm ? L.Rb[c->cur_rb] : L.R[c->iR_cur];
@@ -1263,9 +1273,14 @@ int group_step(GroupRun &g) {
   hipStream_t st = c->st;
   // the pointer arguments are the first member's (its tables serve all)
   HIPCHECK(rism::run_zfwd(P, L.T[ix.iT], L.u, L.fr, L.spec, L.tb.twz, L.tb.zpre, L.tb.zpost, st));
-  HIPCHECK(rism::run_y(P, L.spec, -1, L.tb.twy, L.tb.prey, st));
-  HIPCHECK(rism::run_xoz(P, L.spec, L.fk, L.tb.twx, L.tb.prex, c->knots, c->coef, L.chitab, st));
-  HIPCHECK(rism::run_y(P, L.spec, +1, L.tb.twy, L.tb.prey, st));
+  if (rism::plane_offered(P)) {
+    HIPCHECK(rism::run_plane(P, L.spec, L.fk, L.tb.twx, L.tb.prex, L.tb.twy, L.tb.prey, L.chitab,
+                             st));
+  } else {
+    HIPCHECK(rism::run_y(P, L.spec, -1, L.tb.twy, L.tb.prey, st));
+    HIPCHECK(rism::run_xoz(P, L.spec, L.fk, L.tb.twx, L.tb.prex, c->knots, c->coef, L.chitab, st));
+    HIPCHECK(rism::run_y(P, L.spec, +1, L.tb.twy, L.tb.prey, st));
+  }
   // (in a group the Q, P and slot pointers come from the table)
   HIPCHECK(rism::run_zinv(P, L.spec, L.T[ix.iT], L.u, L.R[ix.iR], (double *)nullptr, L.R[ix.s0],
                           L.R[ix.s1],

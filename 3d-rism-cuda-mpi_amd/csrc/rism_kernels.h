@@ -109,6 +109,12 @@ template <class Re>
 hipError_t run_xoz(const Params &P, cx<Re> *spec, const cx<Re> *fkraw, const cx<Re> *twL,
                    const cx<Re> *prex, const double *knots, const double *coef,
                    const Re *chitab, hipStream_t st);
+// Passes 2 to 4 (both run_y and run_xoz) in one kernel, where plane_offered:
+// a chi table, 2 or 4 sites, and planes of these lengths that fit the LDS.
+bool plane_offered(const Params &P);
+hipError_t run_plane(const Params &P, cplx *spec, const cplx *fkraw, const cplx *twx,
+                     const cplx *prex, const cplx *twy, const cplx *prey, const double *chitab,
+                     hipStream_t st);
 hipError_t run_chi_table(const double *knots, const double *coef, const Params &P,
                          double kscale, size_t nshell, double *out, hipStream_t st);
 // out: natv^2 (nx/2) (ny/2) (nz/2) values, [m][yh][pair][xh]

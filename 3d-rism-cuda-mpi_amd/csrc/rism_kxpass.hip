@@ -14,7 +14,8 @@
 //                    residual R = h + 1 - g, FP64 partial sums of R.R and of
 //                    the AN2 Gram entries                (tr + theta30)
 //
-// followed by an elementwise AN2 update (anderson_cuda.cu:1-22).
+// followed by an elementwise AN2 update (anderson_cuda.cu:1-22).  Planes that
+// fit the LDS take 2 to 4 in one kernel (rism_kplane.h).
 //
 // Transform convention (fft3d.cu:81-163, fft3d_cuda.cu:56-128, with the
 // S = +1 phase): F(k) = dv sum_r f(r) e^{-ik.r}, f(r) = V^-1 sum_k F(k) e^{ik.r},
@@ -27,45 +28,15 @@
 // Data layout: real fields [site][z][y][x] (x fastest) in FP64; spectra
 // [site][m][y][x] complex FP64 with m in [0, nz/2) <-> k_z index m + nz/2.
 
-#include "rism_common.h"
+#include "rism_chi.h"
 
 namespace rism {
 
 // ---------------------------------------------------------------------------
 // 3. DFT along x, OZ with chi_vv(|k|), inverse DFT along x
 // ---------------------------------------------------------------------------
-// chi_vv(|k|) sources for the OZ step.  ChiTable: a table built once per
-// context, one row of natv^2 values per k^2 shell for a cubic box
-// (k_chi_table), or one per point of the octant kx, ky, kz > 0 for a box with
-// different sides (k_chi_octant; |k| has few repeats there).  ChiSpline: the
-// natural cubic spline of the .xvk table evaluated at |k|
-// (solvent_spline.cu:44-55 evaluates the same spline at the same |k| shell
-// values; splint.cc:4-20 picks the interval).
-// The octant table holds natv^2 / 8 words per grid point, which the pass
-// reads once a step, and against it stood four coefficient gathers, a square
-// root and a knot search per k and pair of sites: 144 x 160 x 128, 4 sites,
-// 124 -> 79 us; 72 x 90 x 60, 2 sites, 17 -> 9 us.
-template <class Tb, int STRIDE>
-struct ChiTable {
-  const Tb *row;
-  __device__ __forceinline__ Tb operator()(int pw) const { return row[pw * STRIDE]; }
-};
-// the table's row for the points (+-kx, +-ky) at x index jx < L/2, y index
-// yh < ny/2 and plane m.  Shells are rows of consecutive values; in the
-// octant the x index is fastest, so that neighbouring threads read
-// neighbouring words.
-template <int L, int CHI, class Tb>
-__device__ __forceinline__ auto chi_row(const Tb *tab, const Params &P, int nv2, int jx, int yh,
-                                        int m) {
-  if constexpr (CHI == RISM_CHI_OCTANT) {
-    return ChiTable<Tb, L / 2>{tab + ((size_t)m * (P.ny / 2) + yh) * nv2 * (L / 2) + jx};
-  } else {
-    // |k|^2 = (pi/L)^2 (8 sidx + 3)
-    const long ox = 2 * jx - L + 1, oy = 2 * yh - P.ny + 1, oz = 2 * m + 1;
-    const long sidx = (ox * ox + oy * oy + oz * oz - 3) >> 3;
-    return ChiTable<Tb, 1>{tab + sidx * nv2};
-  }
-}
+// The third chi source, evaluated at |k| (solvent_spline.cu:44-55; splint.cc:4-20
+// picks the interval).
 struct ChiSpline {
   const double *cf;
   double tt;
@@ -149,32 +120,6 @@ __device__ __forceinline__ void oz_row(cx<Re> *lds, int CS, int jx, int L, const
   const int off[2] = {lpad(jx), lpad(jm)};
   const cx<Re> fk[2] = {fkr ? fkr[jx] : cx<Re>{0, 0}, fkr ? fkr[jm] : cx<Re>{0, 0}};
   oz_dispatch<NVMAX, 2>(lds, CS, off, fk, P, X);
-}
-
-// The same contraction with the chi row already in registers (chr[v][w],
-// v, w < NV): used when every thread owns at most kChiPairs (kx, -kx) pairs,
-// so the rows are fetched before the forward transform and their latency is
-// hidden.
-template <int NV, int NVM, class Re>
-__device__ __forceinline__ void oz_points_reg(cx<Re> *lds, int CS, const int (&off)[2],
-                                              const cx<Re> (&fk)[2], const Params &P,
-                                              const Re (&chr)[NVM][NVM]) {
-  cx<Re> c[2][NV];
-#pragma unroll
-  for (int w = 0; w < NV; ++w) {
-#pragma unroll
-    for (int k = 0; k < 2; ++k) c[k][w] = lds[off[k] + w * CS] - (Re)P.qv[w] * fk[k];
-  }
-#pragma unroll
-  for (int v = 0; v < NV; ++v) {
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      cx<Re> a{0, 0};
-#pragma unroll
-      for (int w = 0; w < NV; ++w) a = a + chr[v][w] * c[k][w];
-      lds[off[k] + v * CS] = a;
-    }
-  }
 }
 
 // the first stage's elements of one row, pre-twiddled (zeros for a spare row)

@@ -231,7 +231,7 @@ int rism_run(rism_ctx *ctx, int maxstep, double tol, rism_thermo_out *out,
  * stream; durations accumulate per kernel until the next reset. */
 #define RISM_K_ZFWD 0     /* closure + z forward (real -> half complex)      */
 #define RISM_K_YFWD 1     /* y forward                                        */
-#define RISM_K_XOZ 2      /* x forward + OZ + x inverse                       */
+#define RISM_K_XOZ 2      /* x forward + OZ + x inverse (small planes: y too) */
 #define RISM_K_YINV 3     /* y inverse                                        */
 #define RISM_K_ZINV 4     /* z inverse + residual + Gram partial sums         */
 #define RISM_K_REDUCE 5   /* FP64 column reductions of the partial sums       */
