@@ -167,6 +167,10 @@ constexpr int kChiPairs = NVMAX == 2 ? 2 : 1;
 // pair run side by side in workgroups of their own (64^3, 2 sites, 256 waves
 // in pairs: 9.8 -> 6.5 us, with the 2-site kernel)
 constexpr long kPairedWaves = 2048;
+// threads of a workgroup of several row slots: one pair of 160-point rows of 4
+// sites is 80 threads, 62 % of two waves; three of them fill four to 94 %
+// (160^3, 4 sites: 86.7 -> 76.7 us)
+constexpr int kSlotThreads = 256;
 
 // The FP64 table kernels of up to 4 sites are held to 168 VGPRs, three waves
 // per SIMD (160 points took 170: 86 -> 102 us at 160^3); rows of 36 and 72
@@ -435,8 +439,25 @@ static void launch_xoz(const Params &P, cx<Re> *spec, const cx<Re> *fkraw, const
   // the OZ pass takes the rows in mirror pairs (y, ny-1-y), one after the
   // other, when the pairs are enough workgroups to fill the chip
   const int ngrp = P.grp ? P.ngrp : 1;
-  // short rows: several to a workgroup (row slots), so that it fills a wave
-  const int slots = (FftShape<L>::T >= 64 || threads >= 64) ? 1 : 64 / threads;
+  // short rows: several to a workgroup (row slots), so that it fills a wave,
+  // and in launches that fill the chip as many as leave the fewest lanes idle
+  // in the workgroup's last wave or on spare slots
+  int slots = 1;
+  if constexpr (FftShape<L>::T < 64) {
+    slots = threads >= 64 ? 1 : 64 / threads;
+    const int pairs = (P.ny + 1) / 2;
+    auto lanes = [&](int s) {  // taken by one plane's row pairs
+      return (long)((pairs + s - 1) / s) * ((s * threads + 63) / 64 * 64);
+    };
+    if (lanes(slots) / 64 * (P.nz / 2) * ngrp >= kPairedWaves) {
+      long best = lanes(slots);
+      for (int s = slots + 1; s * threads <= kSlotThreads; ++s)
+        if (lanes(s) * 21 <= best * 20) {
+          best = lanes(s);
+          slots = s;
+        }
+    }
+  }
   const int pthreads = slots * threads;
   const size_t plds = (size_t)slots * lds;
   const long waves = ((pthreads + 63) / 64) * (long)((P.ny / 2 + slots - 1) / slots) *
