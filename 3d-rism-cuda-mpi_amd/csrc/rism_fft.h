@@ -1,4 +1,4 @@
-// rism_fft.h -- LDS-staged mixed-radix (2,3,4,5,8) Stockham FFT of columns,
+// rism_fft.h -- LDS-staged mixed-radix (2,3,4,5,6,8) Stockham FFT of columns,
 // the building block of the axis passes in rism_kernels.hip.
 //
 // One column (a line of L complex values along one grid axis) is transformed
@@ -157,6 +157,25 @@ struct Dft<5, S> {
   }
 };
 
+// 6 = 2 x 3 coprime: outputs (3 a + 4 b) mod 6 of inputs (3 c + 2 d) mod 6 without
+// twiddles in between (the prime-factor map)
+template <int S>
+struct Dft<6, S> {
+  template <class Re>
+  __device__ __forceinline__ static void run(cx<Re> *v) {
+    cx<Re> e[3] = {v[0], v[2], v[4]};
+    cx<Re> o[3] = {v[3], v[5], v[1]};
+    Dft<3, S>::run(e);
+    Dft<3, S>::run(o);
+    v[0] = e[0] + o[0];
+    v[3] = e[0] - o[0];
+    v[4] = e[1] + o[1];
+    v[1] = e[1] - o[1];
+    v[2] = e[2] + o[2];
+    v[5] = e[2] - o[2];
+  }
+};
+
 // ---- compile-time factorisation ------------------------------------------
 struct RadixList {
   int n;
@@ -164,7 +183,13 @@ struct RadixList {
 };
 
 // maxr = 8: as many radix-8 stages as possible; maxr = 4: radix-4 stages
-// (twice the threads per column, smaller butterflies)
+// (twice the threads per column, smaller butterflies); kSixes: radix 6 for pairs
+// of a 2 and a 3 where that makes the plan shorter than with 8: 30 = 6 5, 36 =
+// 6 6, 48 = 8 6, 90 = 6 5 3, 144 = 8 6 3, 180 = 6 6 5.  Half the threads per
+// column or so: not for the x pass (144 points spill 40 VGPRs, 79 -> 101 us) and
+// the residual pass (30 points 17.6 -> 21.3 us), whose outputs each wait for
+// loads.
+constexpr int kSixes = 86;
 constexpr RadixList make_radices(int L, int maxr = 8) {
   RadixList rl{0, {}};
   int m = L;
@@ -185,11 +210,31 @@ constexpr RadixList make_radices(int L, int maxr = 8) {
     }
     twos = (rem == 1 && n4 == 0) ? 1 : 0;
   }
+  int n6 = 0, n5 = 0, n3 = 0;
+  while (m % 5 == 0) { ++n5; m /= 5; }
+  while (m % 3 == 0) { ++n3; m /= 3; }
+  if (maxr == kSixes) {
+    int best = n8 + n4 + twos + n3;
+    const int tw = n8 * 3 + n4 * 2 + twos, th = n3;
+    for (int k = 1; k <= tw && k <= th; ++k) {
+      const int a = (tw - k) / 3, rem = (tw - k) % 3;
+      const int cnt = k + a + (rem != 0) + th - k;
+      if (cnt < best) {
+        best = cnt;
+        n6 = k;
+        n8 = a;
+        n4 = rem == 2;
+        twos = rem == 1;
+        n3 = th - k;
+      }
+    }
+  }
   for (int i = 0; i < n8; ++i) rl.r[rl.n++] = 8;
+  for (int i = 0; i < n6; ++i) rl.r[rl.n++] = 6;
   for (int i = 0; i < n4; ++i) rl.r[rl.n++] = 4;
   for (int i = 0; i < twos; ++i) rl.r[rl.n++] = 2;
-  while (m % 5 == 0) { rl.r[rl.n++] = 5; m /= 5; }
-  while (m % 3 == 0) { rl.r[rl.n++] = 3; m /= 3; }
+  for (int i = 0; i < n5; ++i) rl.r[rl.n++] = 5;
+  for (int i = 0; i < n3; ++i) rl.r[rl.n++] = 3;
   if (m != 1) rl.n = -1;  // unsupported prime factor
   return rl;
 }

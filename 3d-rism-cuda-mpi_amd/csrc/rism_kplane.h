@@ -10,11 +10,12 @@ namespace rism {
 // writes it once; the three passes it stands for move it three times.  The
 // planes fill the LDS (one workgroup per CU from 64 x 64, 2 sites, on), so a
 // stage's LDS accesses, FP64 arithmetic and addresses follow one another: some
-// 2 us a stage, four axis transforms of two or three stages.  64^3, 2 sites: 16.5
-// us, about the time of the three passes and their launches on one grid; in
-// groups of solutes, where the passes are bound by the bytes they move, it gains
-// (48 solutes of 48 to 96 points a side, half their volume in planes that fit, 48
-// steps: 63.8 -> 61.5 ms).
+// 2 us a stage, four axis transforms of two or three stages (radix 6 saves one
+// of 48 points: 14.5 -> 11.5 us at 48^3).  64^3, 2 sites: 16.5 us, about the time
+// of the three passes and their launches on one grid; in groups of solutes,
+// where the passes are bound by the bytes they move, it gains (48 solutes of 48
+// to 96 points a side, half their volume in planes that fit, 48 steps: 63.8 ->
+// 61.5 ms).
 //
 // All butterflies of a stage are shared out over the workgroup, column index
 // fastest: lanes of a wave take neighbouring columns, which sit 1 element (y
@@ -27,10 +28,9 @@ struct Plane {
   static constexpr int RS = LX + 1;                  // row stride
   static constexpr int SS = LY * RS;                 // site stride
   static constexpr int TAB = 2 * (LX + LY);          // the axes' roots and pre-twiddles
-  static constexpr long BYTES = 16L * (NV * SS + TAB);
   // registers (complex values) and work (in waves' rounds) of a stage plan
   static constexpr int held(int L, int ncol, int nt) {
-    const RadixList rl = make_radices(L);
+    const RadixList rl = make_radices(L, kSixes);
     int mx = 0;
     for (int i = 0; i < rl.n; ++i) {
       const int r = rl.r[i], per = (L / r * ncol + nt - 1) / nt;
@@ -39,7 +39,7 @@ struct Plane {
     return mx;
   }
   static constexpr long rounds(int L, int ncol, int nt) {
-    const RadixList rl = make_radices(L);
+    const RadixList rl = make_radices(L, kSixes);
     long w = 0;
     for (int i = 0; i < rl.n; ++i) {
       const int r = rl.r[i];
@@ -83,7 +83,7 @@ struct Plane {
 // meets the one that the tables' writers need.
 template <class A, int NT, int S, int STAGE = 0, int NS = 1, class In, class Out>
 __device__ __forceinline__ void plane_dft(cplx *lds, const cplx *tw, In &in, Out &out) {
-  constexpr RadixList rl = make_radices(A::L);
+  constexpr RadixList rl = make_radices(A::L, kSixes);
   constexpr int R = rl.r[STAGE], NB = A::L / R, TOT = NB * A::NCOL, PER = (TOT + NT - 1) / NT;
   constexpr bool first = STAGE == 0, last = STAGE == rl.n - 1;
   constexpr bool FULL = TOT % NT == 0;
