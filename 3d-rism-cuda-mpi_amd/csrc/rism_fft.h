@@ -1,4 +1,4 @@
-// rism_fft.h -- LDS-staged mixed-radix (2,3,4,5,6,8) Stockham FFT of columns,
+// rism_fft.h -- LDS-staged mixed-radix (2,3,4,5,6,8,9,10) Stockham FFT of columns,
 // the building block of the axis passes in rism_kernels.hip.
 //
 // One column (a line of L complex values along one grid axis) is transformed
@@ -176,6 +176,53 @@ struct Dft<6, S> {
   }
 };
 
+// 10 = 2 x 5 the same way: outputs (5 a + 6 b) mod 10 of inputs (5 c + 2 d) mod 10
+template <int S>
+struct Dft<10, S> {
+  template <class Re>
+  __device__ __forceinline__ static void run(cx<Re> *v) {
+    cx<Re> e[5] = {v[0], v[2], v[4], v[6], v[8]};
+    cx<Re> o[5] = {v[5], v[7], v[9], v[1], v[3]};
+    Dft<5, S>::run(e);
+    Dft<5, S>::run(o);
+#pragma unroll
+    for (int b = 0; b < 5; ++b) {
+      v[(6 * b) % 10] = e[b] + o[b];
+      v[(6 * b + 5) % 10] = e[b] - o[b];
+    }
+  }
+};
+
+// 9 = 3 x 3 with the twiddles w9^(a b)
+template <int S>
+struct Dft<9, S> {
+  template <class Re>
+  __device__ __forceinline__ static void run(cx<Re> *v) {
+    constexpr Re c1 = (Re)0.76604444311897803520, s1 = (Re)0.64278760968653932632;
+    constexpr Re c2 = (Re)0.17364817766693034885, s2 = (Re)0.98480775301220805937;
+    constexpr Re c4 = (Re)-0.93969262078590838405, s4 = (Re)0.34202014332566873304;
+    cx<Re> q[3][3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      q[a][0] = v[a];
+      q[a][1] = v[a + 3];
+      q[a][2] = v[a + 6];
+      Dft<3, S>::run(q[a]);
+    }
+    q[1][1] = cmul(q[1][1], cx<Re>{c1, S * s1});
+    q[1][2] = cmul(q[1][2], cx<Re>{c2, S * s2});
+    q[2][1] = cmul(q[2][1], cx<Re>{c2, S * s2});
+    q[2][2] = cmul(q[2][2], cx<Re>{c4, S * s4});
+#pragma unroll
+    for (int b = 0; b < 3; ++b) {
+      cx<Re> r[3] = {q[0][b], q[1][b], q[2][b]};
+      Dft<3, S>::run(r);
+#pragma unroll
+      for (int a = 0; a < 3; ++a) v[b + 3 * a] = r[a];
+    }
+  }
+};
+
 // ---- compile-time factorisation ------------------------------------------
 struct RadixList {
   int n;
@@ -190,8 +237,19 @@ struct RadixList {
 // the residual pass (30 points 17.6 -> 21.3 us), whose outputs each wait for
 // loads.
 constexpr int kSixes = 86;
+// kTens: the same with two stages of 60 = 10 6, 72 = 9 8 and 80 = 10 8, for
+// kernels with registers for them (plane pass in groups: 60 x 72 31 -> 25 us, 60 x
+// 60 29 -> 23 us, 60 x 80 31 -> 23 us, 72 x 64 the same).
+constexpr int kTens = 106;
+
 constexpr RadixList make_radices(int L, int maxr = 8) {
   RadixList rl{0, {}};
+  if (maxr == kTens) {
+    if (L == 60) return RadixList{2, {10, 6}};
+    if (L == 72) return RadixList{2, {9, 8}};
+    if (L == 80) return RadixList{2, {10, 8}};
+    maxr = kSixes;
+  }
   int m = L;
   int n8 = 0, n4 = 0, n2 = 0;
   while (m % 2 == 0) { ++n2; m /= 2; }
@@ -297,7 +355,7 @@ template <class T>
 struct is_mirror_block<T, std::void_t<typename T::mirror_block>> : std::true_type {};
 
 // w[r] = w[1]^r for r = 2 .. R-1, each by one complex product of lower
-// powers (at most three products deep, so within a few ulps of the
+// powers (at most four products deep, so within a few ulps of the
 // correctly rounded table value).  One table load per butterfly instead of
 // R - 1: the dependent global loads of the twiddles measured 10-20 % of the
 // x and y passes at 512 points.
@@ -309,7 +367,9 @@ __device__ __forceinline__ void twiddle_powers(cx<Re> (&w)[R]) {
   if constexpr (R >= 6) w[5] = cmul(w[4], w[1]);
   if constexpr (R >= 7) w[6] = cmul(w[4], w[2]);
   if constexpr (R >= 8) w[7] = cmul(w[4], w[3]);
-  static_assert(R <= 8, "radix above 8");
+  if constexpr (R >= 9) w[8] = cmul(w[4], w[4]);
+  if constexpr (R >= 10) w[9] = cmul(w[5], w[4]);
+  static_assert(R <= 10, "radix above 10");
 }
 
 // The first powers w1 of one stage's twiddles, one per butterfly of the

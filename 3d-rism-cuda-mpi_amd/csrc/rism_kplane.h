@@ -30,7 +30,7 @@ struct Plane {
   static constexpr int TAB = 2 * (LX + LY);          // the axes' roots and pre-twiddles
   // registers (complex values) and work (in waves' rounds) of a stage plan
   static constexpr int held(int L, int ncol, int nt) {
-    const RadixList rl = make_radices(L, kSixes);
+    const RadixList rl = make_radices(L, kTens);
     int mx = 0;
     for (int i = 0; i < rl.n; ++i) {
       const int r = rl.r[i], per = (L / r * ncol + nt - 1) / nt;
@@ -39,7 +39,7 @@ struct Plane {
     return mx;
   }
   static constexpr long rounds(int L, int ncol, int nt) {
-    const RadixList rl = make_radices(L, kSixes);
+    const RadixList rl = make_radices(L, kTens);
     long w = 0;
     for (int i = 0; i < rl.n; ++i) {
       const int r = rl.r[i];
@@ -54,7 +54,7 @@ struct Plane {
     long bw = -1;
     for (int nt = 1024; nt >= 512; nt -= 64) {
       const int hx = held(LX, NV * LY, nt), hy = held(LY, NV * LX, nt);
-      if ((hx > hy ? hx : hy) > (nt > 768 ? 12 : 16)) continue;
+      if ((hx > hy ? hx : hy) > (nt > 768 ? 12 : 18)) continue;
       const long w = rounds(LX, NV * LY, nt) + rounds(LY, NV * LX, nt);
       if (bw < 0 || w < bw) {
         bw = w;
@@ -83,7 +83,7 @@ struct Plane {
 // meets the one that the tables' writers need.
 template <class A, int NT, int S, int STAGE = 0, int NS = 1, class In, class Out>
 __device__ __forceinline__ void plane_dft(cplx *lds, const cplx *tw, In &in, Out &out) {
-  constexpr RadixList rl = make_radices(A::L, kSixes);
+  constexpr RadixList rl = make_radices(A::L, kTens);
   constexpr int R = rl.r[STAGE], NB = A::L / R, TOT = NB * A::NCOL, PER = (TOT + NT - 1) / NT;
   constexpr bool first = STAGE == 0, last = STAGE == rl.n - 1;
   constexpr bool FULL = TOT % NT == 0;

@@ -1,8 +1,7 @@
 """Small planes take the y, x and inverse y passes in one kernel.  One step of
 it is compared with one step of the three passes, which the spline x pass of
-the same context options runs (chi_spline); both transform the same values with
-radix plans of the same depth, so they agree to rounding: a few hundred ulps of
-the largest value.  Every pair of lengths and site count that the kernel is
+the same context options runs (chi_spline); both transform the same values, so they agree to
+rounding: a few hundred ulps of the largest value.  Every pair of lengths and site count that the kernel is
 built for, the smallest nz, and the nearest grid that does not fit.
 """
 import numpy as np
