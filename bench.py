@@ -162,15 +162,16 @@ def solu_dict(sol):
     return {"usig": sol["sig"], "ueps": sol["eps"], "uq": sol["q"], "uxyz": sol["xyz"]}
 
 
-def algorithmic_bytes(natv, N, hist=2, w=8):
+def algorithmic_bytes(natv, N, hist=0, w=8):
     """Minimal HBM bytes per launch of each hot-loop kernel (w bytes per bulk
-    word) with `hist` history residuals (2 for AN2, m for Anderson(m)):
+    word) with `hist` history pairs of Anderson(m), 0 for AN2:
     zfwd reads t, u (2n) and fr (1), writes the half spectrum (n);
     each y pass reads and writes the spectrum (2n);
     xpass_oz reads the spectrum (n) and the half fk (1), writes (n);
-    zinv reads the spectrum, t, u (3n) and the history residuals (hist n),
-    writes R (n);
-    the update reads t, R and the history P_p (hist n), writes t', P_new (2n)."""
+    zinv reads the spectrum, t, u (3n) and the history residuals (2n or hist n),
+    writes R (n) and, AN2, the mixed iterate Q (n);
+    the AN2 update reads Q, P0, P1 (3n), writes t' (n); Anderson(m)'s reads t, R
+    and the history P_p (hist n), writes t', P_new (2n)."""
     ww = float(w) * N
     n = natv
     return {
@@ -178,8 +179,8 @@ def algorithmic_bytes(natv, N, hist=2, w=8):
         "ypass_fwd": 2 * n * ww,
         "xpass_oz": (2 * n + 1) * ww,
         "ypass_inv": 2 * n * ww,
-        "zinv_resid": (4 + hist) * n * ww,
-        "an2_update": (4 + hist) * n * ww,
+        "zinv_resid": (4 + hist if hist else 7) * n * ww,
+        "an2_update": (4 + hist if hist else 4) * n * ww,
     }
 
 
@@ -295,7 +296,7 @@ def phase_headline(args, budget, R):
         ctx["h64"] = g.fields(rism.FIELD_H)
     ks = kernel_profile(g, args.profile_steps)
     g.close()
-    ab = algorithmic_bytes(natv, N, mh)
+    ab = algorithmic_bytes(natv, N, am)
     R["out"]["config"]["kernels"] = per_kernel_table(ks, ab)
     hot = {k: v for k, v in ks.items() if k in ab}
     dom = max(hot, key=lambda k: hot[k][1])
@@ -351,7 +352,7 @@ def phase_mixed(args, budget, R, ctx):
     s64 = R["out"]["value"]
     N, natv = ctx["N"], ctx["natv"]
     mh = ctx["am"] if ctx["am"] > 0 else 2
-    ab32 = algorithmic_bytes(natv, N, mh, w=4)
+    ab32 = algorithmic_bytes(natv, N, ctx["am"], w=4)
     R["out"]["mixed"] = {
         "s_per_solve": wall / nt, "solves_timed": nt, "warmup": nw,
         "speedup_vs_fp64": s64 / (wall / nt),
@@ -549,7 +550,7 @@ def kernel_key(name):
         return "xpass_oz"
     if "k_zinv_resid" in name:
         return "zinv_resid"
-    if "k_an2_update" in name:
+    if "k_an2_update" in name or "k_an2_mix" in name:
         return "an2_update"
     if "k_andm_update" in name:
         return "an2_update"
