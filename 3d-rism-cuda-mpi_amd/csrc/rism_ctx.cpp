@@ -166,8 +166,7 @@ struct rism_ctx {
   double *partial = nullptr, *tpartial = nullptr, *sums = nullptr, *scratch = nullptr;
   // the solute as run_potential_r takes it: atoms sorted by type
   double *atoms = nullptr, *tdata = nullptr;
-  int *trange = nullptr;
-  int ntype = 0;
+  int *types = nullptr;
   double *knots = nullptr, *coef = nullptr, *chitab = nullptr;
   size_t nchitab = 0;  // doubles in chitab
   size_t zinv_blocks = 0;
@@ -456,10 +455,12 @@ int make_solute(rism_ctx *c) {
   std::vector<int> range(nt + 1, 0);
   for (int t : type) ++range[t + 1];
   for (int t = 0; t < nt; ++t) range[t + 1] += range[t];
-  std::vector<int> at(range.begin(), range.end() - 1);
+  std::vector<int> at(range.begin(), range.end() - 1), sorted(nu);
   std::vector<double> atoms(4 * (size_t)std::max(nu, 1), 0.0);
   for (int a = 0; a < nu; ++a) {
-    double *p = atoms.data() + 4 * (size_t)at[type[a]]++;
+    const int i = at[type[a]]++;
+    sorted[i] = type[a];
+    double *p = atoms.data() + 4 * (size_t)i;
     for (int d = 0; d < 3; ++d) p[d] = c->uxyz[3 * (size_t)a + d];
     p[3] = c->uq[a];
   }
@@ -476,10 +477,9 @@ int make_solute(rism_ctx *c) {
       p[1 + 2 * nv + v] = e4 * s6;
     }
   }
-  c->ntype = nt;
   int rc;
   if ((rc = upload(c, &c->atoms, atoms))) return rc;
-  if ((rc = upload(c, &c->trange, range))) return rc;
+  if ((rc = upload(c, &c->types, sorted))) return rc;
   return upload(c, &c->tdata, data);
 }
 
@@ -1431,7 +1431,7 @@ int setup_enqueue(rism_ctx *c) {
   const int do_coul = c->opts.ad_switch != 1;  // cal_Coulomb.cu:23
   {
     KTime kt(c, RISM_K_POT);
-    HIPCHECK(rism::run_potential_r(c->atoms, c->trange, c->tdata, c->ntype, c->P, ikbt, ubeta,
+    HIPCHECK(rism::run_potential_r(c->atoms, c->types, c->tdata, c->natu, c->P, ikbt, ubeta,
                                    do_coul, c->d.u, c->d.fr, c->st));
   }
   if (do_coul && c->natu > 0) {

@@ -198,9 +198,9 @@ hipError_t run_rebase_down(const double *x, const double *t0, float *out, size_t
                            hipStream_t st);
 // streaming copy of n doubles (n even): reads n, writes n
 hipError_t run_copy(const double *in, double *out, size_t n, hipStream_t st);
-// atoms: x, y, z, q each, sorted by type; type t: atoms [trange[t],
-// trange[t+1]) and 1 + 3 natv values in tdata (rism_kpot.hip)
-hipError_t run_potential_r(const double *atoms, const int *trange, const double *tdata, int ntype,
+// atoms: x, y, z, q each, sorted by type, and the type of each; type t: 1 + 3
+// natv values in tdata (rism_kpot.hip)
+hipError_t run_potential_r(const double *atoms, const int *types, const double *tdata, int natu,
                            const Params &P, double ikbt, double ubeta, int do_coul, double *u,
                            double *fr, hipStream_t st);
 // work: nwork complex of scratch, at least nx/2 + ny + nz/2
