@@ -48,7 +48,10 @@ struct Plane {
     return w;
   }
   // threads: the least work done by spare butterflies, among the counts whose
-  // stages fit the registers (128 of a thread above 768 threads, else 168)
+  // stages hold at most 12 complex values a thread (above 768 threads, which have
+  // 128 registers) or 18 (168 registers).  Where no count passes (60 x 72 and 60 x
+  // 80 either way round, 2 sites; 40 x 60, 4 sites) 1024 threads, which hold the
+  // least, 16 (114 to 126 registers, nothing spilled).
   static constexpr int threads() {
     int best = 1024;
     long bw = -1;
@@ -252,7 +255,15 @@ __global__ void __launch_bounds__((Plane<LX, LY, NV>::NT))
 }
 
 // Which planes the kernel is built for: those that fit the LDS, of the lengths
-// that grids of small molecules take.
+// that grids of small molecules take.  Every grid of such planes takes it, in
+// groups and alone, as a solve must not differ by who shares its launches (the
+// passes' radices and so their rounding differ).  Groups decide: 16 solutes of
+// 72 x 64 x 32, 2 sites, 205 -> 169 us a step, of 48 x 48 x 32, 4 sites, 183 -> 150.
+// Alone, few workgroups (nz / 2) that fill the LDS each leave the chip idle.  A
+// step takes 0.86 to 1.02 of the three passes' time for planes of up to 7200
+// points of all sites, and of larger ones up to 1.00 from nz = 64 on (from nz = 128
+// for 64 x 72, for 48 x 48 with 4 sites, and 1.02 of it for 48 x 96); below, 34.2
+// -> 37.3 us at 64 x 64 x 32 and, the most, 40.5 -> 48.3 us at 96 x 48 x 32.
 #define RISM_PLANE_LENGTHS(X) X(40) X(48) X(60) X(64) X(72) X(80) X(96)
 constexpr bool plane_fits(int nx, int ny, int natv) {
   return 16L * (natv * (long)ny * (nx + 1) + 2 * (nx + ny)) <= 160 * 1024;
