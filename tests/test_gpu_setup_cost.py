@@ -41,3 +41,15 @@ def test_many_types(rism, golden, gpu):
 ])
 def test_own_phases(rism, golden, gpu, grid, natu, ntype, sites):
     potentials.test_potentials(rism, golden, gpu, grid, 0.5, natu, ntype, sites, False)
+
+
+def test_no_atoms(rism, golden, gpu):
+    d = rism.read_xvk(f"{golden}/h2o_vv.xvk")
+    none = np.zeros(0)
+    g = rism.RISM3D((16, 20, 24), (8.0, 10.0, 12.0), d,
+                    {"usig": none, "ueps": none, "uq": none, "uxyz": none})
+    g.initialize()
+    assert not g.fields(rism.FIELD_U).any() and not g.get(rism.FIELD_FR).any()
+    assert not g.fk_half().any()
+    assert g.calculate() == 0.0  # the bulk solvent: h = 0 everywhere
+    g.close()
