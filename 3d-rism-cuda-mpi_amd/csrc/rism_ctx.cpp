@@ -171,12 +171,16 @@ struct rism_ctx {
   size_t nchitab = 0;  // doubles in chitab
   size_t zinv_blocks = 0;
   std::vector<void *> allocs;
+  // optional buffers (namespace spare), null without them: the octant chi
+  // tables and the third AN2 iterates of both levels, each one allocation, so
+  // that a level is never without what the other has
+  void *opt_chi = nullptr, *opt_iterate = nullptr;
   // AN2 state (anderson.h:18-40)
   int count = 0, binary = 0;
   double lastx[2] = {0, 0}, lasts[2] = {0, 0};
   // t ping-pongs between T[0] and T[1]; slot p holds P_p = T_p + m R_p in
   // Pslot[iR_slot[p]] and R_p in R[iR_slot[p]] (rotated by pointer; without
-  // memory for Pslot[2], P_p in Pslot[p]).  The residual pass writes t + m R to
+  // Pslot[2], which is optional, P_p in Pslot[p]).  The residual pass writes t + m R to
   // Pslot[iR_cur]; q_ok: it did for the t and R at hand.
   int iT_cur = 0, iR_cur = 0, iR_slot[2] = {1, 2};
   bool q_ok = false;
@@ -244,23 +248,13 @@ struct rism_ctx {
     *p = (Tp *)q;
     return RISM_OK;
   }
-  void release(void *p) {
-    for (size_t i = 0; i < allocs.size(); ++i)
-      if (allocs[i] == p) {
-        (void)hipFree(p);
-        allocs.erase(allocs.begin() + i);
-        return;
-      }
-  }
-  ~rism_ctx() {
+  void drop_graph() {
     if (gexec) (void)hipGraphExecDestroy(gexec);
     if (graph) (void)hipGraphDestroy(graph);
-    if (hscal) (void)hipHostFree(hscal);
-    if (hflag) (void)hipHostFree(hflag);
-    for (hipEvent_t e : evpool) (void)hipEventDestroy(e);
-    for (void *q : allocs) (void)hipFree(q);
-    if (st) (void)hipStreamDestroy(st);
+    gexec = nullptr;
+    graph = nullptr;
   }
+  ~rism_ctx();
 };
 
 namespace {
@@ -274,7 +268,39 @@ template <>
 Level<float> &lv<float>(rism_ctx *c) {
   return c->f;
 }
+
+// P of AN2 slot p
+template <class Re>
+Re *slot_iterate(const rism_ctx *c, const Level<Re> &L, int p) {
+  return L.Pslot[2] ? L.Pslot[c->iR_slot[p]] : L.Pslot[p];
+}
 }  // namespace
+
+// ---- optional buffers --------------------------------------------------------
+// Two buffers make a step shorter but can be done without: the octant chi table
+// of a box with different sides (else the x pass evaluates the spline) and the
+// third AN2 iterate (else the update forms it).
+namespace spare {
+void *take(size_t bytes) {
+  void *q = nullptr;
+  if (hipMalloc(&q, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  return q;
+}
+}  // namespace spare
+
+rism_ctx::~rism_ctx() {
+  drop_graph();
+  if (hscal) (void)hipHostFree(hscal);
+  if (hflag) (void)hipHostFree(hflag);
+  for (hipEvent_t e : evpool) (void)hipEventDestroy(e);
+  for (void *q : allocs) (void)hipFree(q);
+  if (opt_chi) (void)hipFree(opt_chi);
+  if (opt_iterate) (void)hipFree(opt_iterate);
+  if (st) (void)hipStreamDestroy(st);
+}
 
 namespace {
 
@@ -401,22 +427,34 @@ int make_chi(rism_ctx *c, const rism_solvent *s) {
   return RISM_OK;
 }
 
-// The octant table of a box with different sides, for both levels.  It is
-// allocated after everything that the context needs; without memory for it
-// the x pass evaluates the spline.
+// The octant table of a box with different sides, for both levels (optional).
 int make_chi_octant(rism_ctx *c) {
   if (c->opts.chi_spline || c->P.shell != RISM_CHI_SPLINE) return RISM_OK;
   const size_t n = (size_t)(c->nx / 2) * (c->ny / 2) * (c->nz / 2) * c->natv * c->natv;
-  double *tab = nullptr;
-  float *tab32 = nullptr;
-  if (c->alloc(&tab, n) || (c->opts.precision == 1 && c->alloc(&tab32, n))) return RISM_OK;
+  const bool both = c->opts.precision == 1;
+  double *tab = (double *)spare::take(n * (sizeof(double) + (both ? sizeof(float) : 0)));
+  if (!tab) return RISM_OK;
+  c->opt_chi = tab;
   HIPCHECK(rism::run_chi_octant(c->knots, c->coef, c->P, tab, c->st));
-  if (tab32) HIPCHECK(rism::run_convert((const double *)tab, tab32, n, c->st));
   c->d.chitab = c->chitab = tab;
-  c->f.chitab = tab32;
+  if (both) {
+    c->f.chitab = (float *)(tab + n);
+    HIPCHECK(rism::run_convert((const double *)tab, c->f.chitab, n, c->st));
+  }
   c->nchitab = n;
   c->P.shell = RISM_CHI_OCTANT;
   return RISM_OK;
+}
+
+// The third AN2 iterate of both levels (optional).
+void make_third_iterate(rism_ctx *c) {
+  if (c->opts.anderson_m > 0) return;
+  const size_t nn = c->N * c->natv;
+  const bool both = c->opts.precision == 1;
+  c->opt_iterate = spare::take(nn * (sizeof(double) + (both ? sizeof(float) : 0)));
+  if (!c->opt_iterate) return;
+  c->d.Pslot[2] = (double *)c->opt_iterate;
+  if (both) c->f.Pslot[2] = (float *)(c->d.Pslot[2] + nn);
 }
 
 int check_sizes(int nx, int ny, int nz, int natv) {
@@ -548,12 +586,6 @@ struct KTime {
     c->pending.push_back({id, a, b});
   }
 };
-
-// P of AN2 slot p
-template <class Re>
-Re *slot_iterate(const rism_ctx *c, const Level<Re> &L, int p) {
-  return L.Pslot[2] ? L.Pslot[c->iR_slot[p]] : L.Pslot[p];
-}
 
 // One Anderson(m) step: the first an2_count steps are the reference's
 // Picard steps t' = t + R (anderson.cu:54-60); after that
@@ -1002,10 +1034,7 @@ int ensure_graph(rism_ctx *c, double tol) {
   const rism_ctx::GraphKey key{c->iT_cur, c->iR_cur, c->iR_slot[0], c->iR_slot[1], c->binary,
                                c->prec, tol, c->rms_hist};
   if (c->gexec && key == c->gkey) return RISM_OK;
-  if (c->gexec) (void)hipGraphExecDestroy(c->gexec);
-  if (c->graph) (void)hipGraphDestroy(c->graph);
-  c->gexec = nullptr;
-  c->graph = nullptr;
+  c->drop_graph();
   // capture from the current state, then restore it (capture runs nothing)
   const int sT = c->iT_cur, sR = c->iR_cur, s0 = c->iR_slot[0], s1 = c->iR_slot[1],
             sb = c->binary, scount = c->count;
@@ -1801,12 +1830,7 @@ rism_ctx *rism_create(const rism_grid *grid, const rism_solvent *solvent,
       hipHostMalloc((void **)&c->hflag, 3 * sizeof(int)) != hipSuccess)
     return fail(rism::set_error(RISM_ERR_NOMEM, "hipHostMalloc failed"));
   if ((rc = make_chi_octant(c))) return fail(rc);
-  // the third AN2 iterate; without memory for it the update forms it itself
-  if (c->opts.anderson_m == 0 && !c->alloc(&c->d.Pslot[2], nn) && c->opts.precision == 1 &&
-      c->alloc(&c->f.Pslot[2], nn)) {
-    c->release(c->d.Pslot[2]);
-    c->d.Pslot[2] = nullptr;
-  }
+  make_third_iterate(c);
   if (tune::enabled() || tune::forced(0) >= 0) {
     if ((rc = tune_level<double>(c))) return fail(rc);
     if (c->opts.precision == 1 && (rc = tune_level<float>(c))) return fail(rc);
@@ -2220,8 +2244,9 @@ int rism_solve_batch(rism_ctx **ctx, int n, int maxstep, double tol, int threads
 int rism_run_batch(rism_ctx **ctx, int n, int maxstep, double tol, int threads,
                    rism_thermo_out *out, int *status, int *steps) {
   if (!ctx || n < 0) return rism::set_error(RISM_ERR_ARG, "null argument");
-  for (int i = 0; i < n; ++i) {
+  for (int i = 0; i < n; ++i)
     if (!ctx[i]) return rism::set_error(RISM_ERR_ARG, "null context in batch");
+  for (int i = 0; i < n; ++i) {
     int rc = setup_enqueue(ctx[i]);
     if (rc) return rc;
   }
