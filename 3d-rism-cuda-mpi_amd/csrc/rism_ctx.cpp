@@ -147,6 +147,10 @@ int rism::set_error(int code, const std::string &msg) {
   return code;
 }
 
+// hipMalloc; when the device has no room, the optional buffers of idle contexts
+// are given back first (and those of `self`, whose caller is between steps)
+static hipError_t device_malloc(void **p, size_t bytes, rism_ctx *self = nullptr);
+
 struct rism_ctx {
   int dev = 0;
   hipStream_t st = nullptr;
@@ -175,6 +179,7 @@ struct rism_ctx {
   // tables and the third AN2 iterates of both levels, each one allocation, so
   // that a level is never without what the other has
   void *opt_chi = nullptr, *opt_iterate = nullptr;
+  int users = 0;  // calls at work on the context, under spare::lock()
   // AN2 state (anderson.h:18-40)
   int count = 0, binary = 0;
   double lastx[2] = {0, 0}, lasts[2] = {0, 0};
@@ -235,12 +240,12 @@ struct rism_ctx {
   std::vector<Pending> pending;
   rism_kstat kstat[RISM_K_COUNT] = {};
 
+  // self: as device_malloc's
   template <class Tp>
-  int alloc(Tp **p, size_t count_elems) {
+  int alloc(Tp **p, size_t count_elems, rism_ctx *self = nullptr) {
     void *q = nullptr;
     const size_t bytes = sizeof(Tp) * (count_elems ? count_elems : 1);
-    if (hipMalloc(&q, bytes) != hipSuccess) {
-      (void)hipGetLastError();
+    if (device_malloc(&q, bytes, self) != hipSuccess) {
       return rism::set_error(RISM_ERR_NOMEM,
                              "hipMalloc of " + std::to_string(bytes) + " bytes failed");
     }
@@ -279,19 +284,152 @@ Re *slot_iterate(const rism_ctx *c, const Level<Re> &L, int p) {
 // ---- optional buffers --------------------------------------------------------
 // Two buffers make a step shorter but can be done without: the octant chi table
 // of a box with different sides (else the x pass evaluates the spline) and the
-// third AN2 iterate (else the update forms it).
+// third AN2 iterate (else the update forms it).  Each adds up to a tenth to a
+// context, so that nothing may fail for their sake:
+//  * a context takes them last, and only while half of the device's memory stays
+//    free, for other libraries and processes;
+//  * an allocation of this library that finds no room gives back those of every
+//    idle context of the device and tries again.  A context is idle while no call
+//    is at work on it (Use), whatever its state between two calls;
+//  * RISM_OPTIONAL_BUFFERS=0 (environment) withholds them.
 namespace spare {
+// (never destroyed: contexts may be, after this library's statics)
+std::mutex &lock() {
+  static std::mutex *m = new std::mutex;
+  return *m;
+}
+std::vector<rism_ctx *> &holders() {  // under lock()
+  static std::vector<rism_ctx *> *v = new std::vector<rism_ctx *>;
+  return *v;
+}
+
 void *take(size_t bytes) {
+  const char *e = std::getenv("RISM_OPTIONAL_BUFFERS");
+  if (e && e[0] == '0') return nullptr;
+  size_t free_b = 0, total = 0;
   void *q = nullptr;
+  if (hipMemGetInfo(&free_b, &total) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  if (free_b < bytes || free_b - bytes < total / 2) return nullptr;
   if (hipMalloc(&q, bytes) != hipSuccess) {
     (void)hipGetLastError();
     return nullptr;
   }
   return q;
 }
+
+void hold(rism_ctx *c) {
+  if (!c->opt_chi && !c->opt_iterate) return;
+  std::lock_guard<std::mutex> g(lock());
+  holders().push_back(c);
+}
+
+void forget(rism_ctx *c) {
+  std::lock_guard<std::mutex> g(lock());
+  auto &h = holders();
+  for (size_t i = 0; i < h.size(); ++i)
+    if (h[i] == c) {
+      h.erase(h.begin() + i);
+      return;
+    }
+}
+
+// The slots' P of a level into Pslot[0] and Pslot[1]; that which is in the third
+// buffer moves to the one that holds none.
+template <class Re>
+hipError_t settle(rism_ctx *c, Level<Re> &L) {
+  if (!L.Pslot[2]) return hipSuccess;
+  Re *P[2] = {slot_iterate(c, L, 0), slot_iterate(c, L, 1)};
+  for (Re *&p : P)
+    if (p == L.Pslot[2]) {
+      Re *to = L.Pslot[c->iR_cur];
+      const hipError_t e = hipMemcpyAsync(to, p, sizeof(Re) * c->N * c->natv,
+                                          hipMemcpyDeviceToDevice, c->st);
+      if (e != hipSuccess) return e;
+      p = to;
+    }
+  L.Pslot[0] = P[0];
+  L.Pslot[1] = P[1];
+  L.Pslot[2] = nullptr;
+  return hipSuccess;
+}
+
+// leaves an idle context as it would be without the optional buffers
+bool drop(rism_ctx *c) {
+  if (hipStreamSynchronize(c->st) != hipSuccess) return false;
+  c->drop_graph();  // its nodes hold the buffers' addresses
+  if (c->opt_iterate) {
+    if (settle(c, c->d) != hipSuccess || settle(c, c->f) != hipSuccess ||
+        hipStreamSynchronize(c->st) != hipSuccess)
+      return false;
+    c->q_ok = false;
+    (void)hipFree(c->opt_iterate);
+    c->opt_iterate = nullptr;
+  }
+  if (c->opt_chi) {
+    c->P.shell = RISM_CHI_SPLINE;
+    c->chitab = c->d.chitab = nullptr;
+    c->f.chitab = nullptr;
+    c->nchitab = 0;
+    (void)hipFree(c->opt_chi);
+    c->opt_chi = nullptr;
+  }
+  return true;
+}
+
+// whether any memory of the current device was given back
+bool give_back(rism_ctx *self) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  std::lock_guard<std::mutex> g(lock());
+  auto &h = holders();
+  bool any = false;
+  for (size_t i = 0; i < h.size();) {
+    rism_ctx *c = h[i];
+    if (c->dev == dev && c->users == (c == self ? 1 : 0) && drop(c)) {
+      h.erase(h.begin() + i);
+      any = true;
+    } else {
+      ++i;
+    }
+  }
+  return any;
+}
+
+// a call at work on n contexts: their optional buffers stay
+struct UseAll {
+  rism_ctx *const *c;
+  int n;
+  UseAll(rism_ctx *const *c_, int n_) : c(c_), n(n_) { add(1); }
+  ~UseAll() { add(-1); }
+  UseAll(const UseAll &) = delete;
+  UseAll &operator=(const UseAll &) = delete;
+  void add(int k) const {
+    std::lock_guard<std::mutex> g(lock());
+    for (int i = 0; i < n; ++i) c[i]->users += k;
+  }
+};
+struct Use {
+  rism_ctx *c;
+  UseAll all;
+  explicit Use(rism_ctx *c_) : c(c_), all(&c, 1) {}
+};
 }  // namespace spare
 
+static hipError_t device_malloc(void **p, size_t bytes, rism_ctx *self) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    if (spare::give_back(self) && (e = hipMalloc(p, bytes)) != hipSuccess)
+      (void)hipGetLastError();
+  }
+  return e;
+}
+
 rism_ctx::~rism_ctx() {
+  spare::forget(this);
   drop_graph();
   if (hscal) (void)hipHostFree(hscal);
   if (hflag) (void)hipHostFree(hflag);
@@ -994,7 +1132,8 @@ bool async_capable(const rism_ctx *c) {
   return c->opts.precision == 0 && !c->opts.verbose;
 }
 
-int async_begin(AsyncRun &a, rism_ctx *c, int maxstep, double tol) {
+// (self: as device_malloc's)
+int async_begin(AsyncRun &a, rism_ctx *c, int maxstep, double tol, rism_ctx *self = nullptr) {
   a = AsyncRun{};
   a.c = c;
   a.maxstep = maxstep;
@@ -1002,7 +1141,7 @@ int async_begin(AsyncRun &a, rism_ctx *c, int maxstep, double tol) {
   a.log.assign(maxstep + 1, AsyncRun::Log{0, 0, 0, 0, 0, 0, 0, 0, {}});
   if (c->rms_cap < (size_t)maxstep + 1) {
     size_t cap = std::max<size_t>(1024, (size_t)maxstep + 1);
-    int rc = c->alloc(&c->rms_hist, cap);
+    int rc = c->alloc(&c->rms_hist, cap, self);
     if (rc) return rc;
     c->rms_cap = cap;
   }
@@ -1276,7 +1415,7 @@ int group_tables(GroupRun &g) {
     }
     ix = group_next(ix);
   }
-  if (hipMalloc(&g.dtab, sizeof(rism::GroupPtrs) * h.size()) != hipSuccess)
+  if (device_malloc((void **)&g.dtab, sizeof(rism::GroupPtrs) * h.size()) != hipSuccess)
     return rism::set_error(RISM_ERR_NOMEM, "hipMalloc of the group tables failed");
   hipStream_t st = g.c0()->st;
   HIPCHECK(hipMemcpyAsync(g.dtab, h.data(), sizeof(rism::GroupPtrs) * h.size(),
@@ -1839,6 +1978,7 @@ rism_ctx *rism_create(const rism_grid *grid, const rism_solvent *solvent,
   if (hipMemsetAsync(c->d.T[0], 0, sizeof(double) * nn, c->st) != hipSuccess ||
       hipStreamSynchronize(c->st) != hipSuccess)
     return fail(rism::set_error(RISM_ERR_HIP, "initial clear failed"));
+  spare::hold(c);
   return c;
 }
 
@@ -1846,6 +1986,7 @@ void rism_destroy(rism_ctx *ctx) { delete ctx; }
 
 int rism_setup_potentials(rism_ctx *c) {
   if (!c) return rism::set_error(RISM_ERR_ARG, "null context");
+  spare::Use use(c);
   int rc = setup_enqueue(c);
   if (rc) return rc;
   HIPCHECK(hipStreamSynchronize(c->st));
@@ -1854,11 +1995,13 @@ int rism_setup_potentials(rism_ctx *c) {
 
 int rism_calculate(rism_ctx *c, double *rms) {
   if (!c) return rism::set_error(RISM_ERR_ARG, "null context");
+  spare::Use use(c);
   return c->prec ? calc_step<float>(c, rms) : calc_step<double>(c, rms);
 }
 
 int rism_anderson(rism_ctx *c) {
   if (!c) return rism::set_error(RISM_ERR_ARG, "null context");
+  spare::Use use(c);
   if (!c->have_step || !c->fresh || c->last_prec != c->prec)
     return rism::set_error(RISM_ERR_STATE, "rism_anderson needs a preceding rism_calculate");
   c->fresh = false;
@@ -1869,6 +2012,7 @@ int rism_anderson(rism_ctx *c) {
 
 int rism_set_precision(rism_ctx *c, int prec) {
   if (!c) return rism::set_error(RISM_ERR_ARG, "null context");
+  spare::Use use(c);
   if (prec != 0 && prec != 1) return rism::set_error(RISM_ERR_ARG, "precision must be 0 or 1");
   if (prec == 1 && c->opts.precision != 1)
     return rism::set_error(RISM_ERR_STATE, "the context was created without the FP32 level");
@@ -1889,10 +2033,11 @@ static bool sync_free_allowed() {
 
 int rism_solve(rism_ctx *c, int maxstep, double tol, int *status, int *steps, double *rms_out) {
   if (!c) return rism::set_error(RISM_ERR_ARG, "null context");
+  spare::Use use(c);
   if (async_capable(c) && !c->ktime && c->prec == 0 && maxstep > 0 && sync_free_allowed()) {
     // same steps without a host round trip per step
     AsyncRun a;
-    int rc = async_begin(a, c, maxstep, tol);
+    int rc = async_begin(a, c, maxstep, tol, c);
     while (!rc && !a.finished) {
       rc = async_enqueue<double>(a, kAsyncChunk);
       if (!rc && hipStreamSynchronize(c->st) != hipSuccess)
@@ -1968,6 +2113,7 @@ int rism_solve(rism_ctx *c, int maxstep, double tol, int *status, int *steps, do
 
 int rism_thermo(rism_ctx *c, rism_thermo_out *out) {
   if (!c || !out) return rism::set_error(RISM_ERR_ARG, "null argument");
+  spare::Use use(c);
   if (!c->have_step) return rism::set_error(RISM_ERR_STATE, "rism_thermo needs a solved state");
   const int tb = rism::thermo_blocks(c->N);
   {
@@ -2019,6 +2165,7 @@ int rism_thermo(rism_ctx *c, rism_thermo_out *out) {
 
 int rism_get_field(rism_ctx *c, int which, int site, double *host) {
   if (!c || !host) return rism::set_error(RISM_ERR_ARG, "null argument");
+  spare::Use use(c);
   if (which != RISM_FIELD_FR && (site < 0 || site >= c->natv))
     return rism::set_error(RISM_ERR_ARG, "site out of range");
   const size_t off = (size_t)site * c->N;
@@ -2078,6 +2225,7 @@ int rism_get_field(rism_ctx *c, int which, int site, double *host) {
 
 int rism_set_field(rism_ctx *c, int which, int site, const double *host) {
   if (!c || !host) return rism::set_error(RISM_ERR_ARG, "null argument");
+  spare::Use use(c);
   if (site < 0 || site >= c->natv) return rism::set_error(RISM_ERR_ARG, "site out of range");
   const size_t off = (size_t)site * c->N;
   if (which == RISM_FIELD_T) {
@@ -2119,6 +2267,7 @@ int rism_solve_batch(rism_ctx **ctx, int n, int maxstep, double tol, int threads
   }
   if (maxstep <= 0) return rism::set_error(RISM_ERR_ARG, "maxstep must be positive");
   if (n == 0) return RISM_OK;
+  const spare::UseAll use(ctx, n);  // groups stay alike
   std::vector<AsyncRun> runs(n);
   const int nt = std::max(1, std::min(threads > 0 ? threads : 1, n));
   std::vector<int> rcs(nt, RISM_OK);
@@ -2246,6 +2395,7 @@ int rism_run_batch(rism_ctx **ctx, int n, int maxstep, double tol, int threads,
   if (!ctx || n < 0) return rism::set_error(RISM_ERR_ARG, "null argument");
   for (int i = 0; i < n; ++i)
     if (!ctx[i]) return rism::set_error(RISM_ERR_ARG, "null context in batch");
+  const spare::UseAll use(ctx, n);
   for (int i = 0; i < n; ++i) {
     int rc = setup_enqueue(ctx[i]);
     if (rc) return rc;
@@ -2355,6 +2505,7 @@ int rism_write_huv(rism_ctx *c, const char *path) { return write_text_field(c, p
 
 int rism_analysis(rism_ctx *c, int kind, double *out) {
   if (!c || !out) return rism::set_error(RISM_ERR_ARG, "null argument");
+  spare::Use use(c);
   if (kind < RISM_ANALYSIS_GRAD || kind > RISM_ANALYSIS_AD)
     return rism::set_error(RISM_ERR_ARG, "unknown analysis kind");
   if (!c->have_step || c->last_prec != 0)
@@ -2392,10 +2543,9 @@ int rism_analysis(rism_ctx *c, int kind, double *out) {
     if (dpart) (void)hipFree(dpart);
     if (dout) (void)hipFree(dout);
   };
-  if (hipMalloc(&dad, sizeof(double) * adata.size()) != hipSuccess ||
-      hipMalloc(&dpart, sizeof(double) * nslab * nu * width) != hipSuccess ||
-      hipMalloc(&dout, sizeof(double) * nu * width) != hipSuccess) {
-    (void)hipGetLastError();
+  if (device_malloc((void **)&dad, sizeof(double) * adata.size(), c) != hipSuccess ||
+      device_malloc((void **)&dpart, sizeof(double) * nslab * nu * width, c) != hipSuccess ||
+      device_malloc((void **)&dout, sizeof(double) * nu * width, c) != hipSuccess) {
     cleanup();
     return rism::set_error(RISM_ERR_NOMEM, "hipMalloc failed in rism_analysis");
   }
@@ -2558,6 +2708,7 @@ int rism_k_fft_c2r(int nx, int ny, int nz, const double box[3], const double *in
 
 int rism_k_get_fk(rism_ctx *c, double *out) {
   if (!c || !out) return rism::set_error(RISM_ERR_ARG, "null argument");
+  spare::Use use(c);
   cplx *tmp = c->d.spec;  // borrow the spectrum buffer
   HIPCHECK(hipMemcpyAsync(tmp, c->d.fk, sizeof(cplx) * (c->N / 2), hipMemcpyDeviceToDevice, c->st));
   HIPCHECK(rism::run_apply_phase(tmp, c->P, c->st));
@@ -2573,9 +2724,8 @@ int rism_k_copy_bench(size_t bytes, int reps, double *avg_ms) {
   hipStream_t st = nullptr;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   int rc = RISM_OK;
-  if (hipMalloc((void **)&a, n * sizeof(double)) != hipSuccess ||
-      hipMalloc((void **)&b, n * sizeof(double)) != hipSuccess) {
-    (void)hipGetLastError();
+  if (device_malloc((void **)&a, n * sizeof(double)) != hipSuccess ||
+      device_malloc((void **)&b, n * sizeof(double)) != hipSuccess) {
     rc = rism::set_error(RISM_ERR_NOMEM, "hipMalloc failed in rism_k_copy_bench");
   }
   if (!rc && (hipStreamCreate(&st) != hipSuccess || hipEventCreate(&e0) != hipSuccess ||

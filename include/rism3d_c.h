@@ -152,7 +152,12 @@ const char *rism_last_error(void);
 /* Replaces RISM3D::initialize (initialize.cu:4-44) up to, not including,
  * cal_potential: uploads the solute, builds the k-grid shells and the chi
  * spline table (initialize_g.cu:7-50, solvent_spline.cu:7-96) and allocates
- * every device buffer.  Returns NULL and sets *err on failure. */
+ * every device buffer.  Returns NULL and sets *err on failure.  Two buffers
+ * that shorten a step but can be done without (a chi_vv table of boxes with
+ * different sides, a third AN2 iterate) are taken only while half of the
+ * device's memory stays free, and are given back by contexts that no call is
+ * at work on when an allocation of this library finds no room; results then
+ * differ in rounding.  RISM_OPTIONAL_BUFFERS=0 (environment) withholds them. */
 rism_ctx *rism_create(const rism_grid *grid, const rism_solvent *solvent,
                       const rism_solute *solute, const rism_opts *opts, int *err);
 /* Frees the context and all its device memory. */
