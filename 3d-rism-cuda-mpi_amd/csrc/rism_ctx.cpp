@@ -919,8 +919,8 @@ int convert_state(rism_ctx *c) {
   int rc;
   for (int i = 0; i < 2; ++i)
     if ((rc = cv(A.T[i], B.T[i]))) return rc;
-  for (int i = 0; i < 3; ++i)
-    if ((rc = cv(A.Pslot[i], B.Pslot[i]))) return rc;
+  for (int p = 0; p < 2; ++p)  // (a third iterate is the next step's, and formed anew)
+    if ((rc = cv(slot_iterate(c, A, p), slot_iterate(c, B, p)))) return rc;
   for (int i = 0; i < 3; ++i)
     if ((rc = cv(A.R[i], B.R[i]))) return rc;
   for (size_t i = 0; i < A.Rb.size(); ++i)
