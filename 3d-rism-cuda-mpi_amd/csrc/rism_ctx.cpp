@@ -1,5 +1,6 @@
 // rism_ctx.cpp -- the C ABI (include/rism3d_c.h): context, set-up, the
-// fixed-point loop, AN2 and the thermodynamics, driving rism_kernels.hip.
+// fixed-point loop, AN2 and the thermodynamics, driving the kernels of
+// rism_k*.hip.
 //
 // Host-side counterpart of the reference's RISM3D orchestration
 // (initialize.cu, iterate.cu, calculate.cu, anderson.cu, output.cu) for one
@@ -175,10 +176,10 @@ struct rism_ctx {
   size_t nchitab = 0;  // doubles in chitab
   size_t zinv_blocks = 0;
   std::vector<void *> allocs;
-  // optional buffers (namespace spare), null without them: the octant chi
-  // tables and the third AN2 iterates of both levels, each one allocation, so
-  // that a level is never without what the other has
-  void *opt_chi = nullptr, *opt_iterate = nullptr;
+  // optional buffers (namespace spare), null without them: the third AN2
+  // iterates and the octant chi tables of both levels, one allocation, so that a
+  // level is never without what the other has
+  void *optional = nullptr;
   int users = 0;  // calls at work on the context, under spare::lock()
   // AN2 state (anderson.h:18-40)
   int count = 0, binary = 0;
@@ -321,7 +322,7 @@ void *take(size_t bytes) {
 }
 
 void hold(rism_ctx *c) {
-  if (!c->opt_chi && !c->opt_iterate) return;
+  if (!c->optional) return;
   std::lock_guard<std::mutex> g(lock());
   holders().push_back(c);
 }
@@ -360,22 +361,18 @@ hipError_t settle(rism_ctx *c, Level<Re> &L) {
 bool drop(rism_ctx *c) {
   if (hipStreamSynchronize(c->st) != hipSuccess) return false;
   c->drop_graph();  // its nodes hold the buffers' addresses
-  if (c->opt_iterate) {
-    if (settle(c, c->d) != hipSuccess || settle(c, c->f) != hipSuccess ||
-        hipStreamSynchronize(c->st) != hipSuccess)
-      return false;
-    c->q_ok = false;
-    (void)hipFree(c->opt_iterate);
-    c->opt_iterate = nullptr;
-  }
-  if (c->opt_chi) {
+  if (settle(c, c->d) != hipSuccess || settle(c, c->f) != hipSuccess ||
+      hipStreamSynchronize(c->st) != hipSuccess)
+    return false;
+  c->q_ok = false;
+  if (c->P.shell == RISM_CHI_OCTANT) {
     c->P.shell = RISM_CHI_SPLINE;
     c->chitab = c->d.chitab = nullptr;
     c->f.chitab = nullptr;
     c->nchitab = 0;
-    (void)hipFree(c->opt_chi);
-    c->opt_chi = nullptr;
   }
+  (void)hipFree(c->optional);
+  c->optional = nullptr;
   return true;
 }
 
@@ -435,8 +432,7 @@ rism_ctx::~rism_ctx() {
   if (hflag) (void)hipHostFree(hflag);
   for (hipEvent_t e : evpool) (void)hipEventDestroy(e);
   for (void *q : allocs) (void)hipFree(q);
-  if (opt_chi) (void)hipFree(opt_chi);
-  if (opt_iterate) (void)hipFree(opt_iterate);
+  if (optional) (void)hipFree(optional);
   if (st) (void)hipStreamDestroy(st);
 }
 
@@ -565,34 +561,41 @@ int make_chi(rism_ctx *c, const rism_solvent *s) {
   return RISM_OK;
 }
 
-// The octant table of a box with different sides, for both levels (optional).
-int make_chi_octant(rism_ctx *c) {
-  if (c->opts.chi_spline || c->P.shell != RISM_CHI_SPLINE) return RISM_OK;
-  const size_t n = (size_t)(c->nx / 2) * (c->ny / 2) * (c->nz / 2) * c->natv * c->natv;
+// The optional buffers: the third AN2 iterate and, for a box with different
+// sides, the octant table, of both levels.
+int make_optional(rism_ctx *c) {
   const bool both = c->opts.precision == 1;
-  double *tab = (double *)spare::take(n * (sizeof(double) + (both ? sizeof(float) : 0)));
-  if (!tab) return RISM_OK;
-  c->opt_chi = tab;
-  HIPCHECK(rism::run_chi_octant(c->knots, c->coef, c->P, tab, c->st));
-  c->d.chitab = c->chitab = tab;
-  if (both) {
-    c->f.chitab = (float *)(tab + n);
-    HIPCHECK(rism::run_convert((const double *)tab, c->f.chitab, n, c->st));
-  }
-  c->nchitab = n;
-  c->P.shell = RISM_CHI_OCTANT;
-  return RISM_OK;
-}
-
-// The third AN2 iterate of both levels (optional).
-void make_third_iterate(rism_ctx *c) {
-  if (c->opts.anderson_m > 0) return;
+  const bool iterate = c->opts.anderson_m == 0;
+  const bool table = !c->opts.chi_spline && c->P.shell == RISM_CHI_SPLINE;
+  if (!iterate && !table) return RISM_OK;
   const size_t nn = c->N * c->natv;
-  const bool both = c->opts.precision == 1;
-  c->opt_iterate = spare::take(nn * (sizeof(double) + (both ? sizeof(float) : 0)));
-  if (!c->opt_iterate) return;
-  c->d.Pslot[2] = (double *)c->opt_iterate;
-  if (both) c->f.Pslot[2] = (float *)(c->d.Pslot[2] + nn);
+  const size_t n = (size_t)(c->nx / 2) * (c->ny / 2) * (c->nz / 2) * c->natv * c->natv;
+  size_t bytes = 0;
+  auto part = [&](bool want, size_t size) {  // offset of one, on a line of its own
+    const size_t at = bytes;
+    if (want) bytes += (size + 255) / 256 * 256;
+    return at;
+  };
+  const size_t it64 = part(iterate, nn * sizeof(double));
+  const size_t it32 = part(iterate && both, nn * sizeof(float));
+  const size_t tab64 = part(table, n * sizeof(double));
+  const size_t tab32 = part(table && both, n * sizeof(float));
+  char *q = (char *)spare::take(bytes);
+  if (!q) return RISM_OK;
+  c->optional = q;
+  if (iterate) c->d.Pslot[2] = (double *)(q + it64);
+  if (iterate && both) c->f.Pslot[2] = (float *)(q + it32);
+  if (table) {
+    c->d.chitab = c->chitab = (double *)(q + tab64);
+    HIPCHECK(rism::run_chi_octant(c->knots, c->coef, c->P, c->chitab, c->st));
+    if (both) {
+      c->f.chitab = (float *)(q + tab32);
+      HIPCHECK(rism::run_convert((const double *)c->chitab, c->f.chitab, n, c->st));
+    }
+    c->nchitab = n;
+    c->P.shell = RISM_CHI_OCTANT;
+  }
+  return RISM_OK;
 }
 
 int check_sizes(int nx, int ny, int nz, int natv) {
@@ -1968,8 +1971,7 @@ rism_ctx *rism_create(const rism_grid *grid, const rism_solvent *solvent,
   if (hipHostMalloc((void **)&c->hscal, 8 * sizeof(double)) != hipSuccess ||
       hipHostMalloc((void **)&c->hflag, 3 * sizeof(int)) != hipSuccess)
     return fail(rism::set_error(RISM_ERR_NOMEM, "hipHostMalloc failed"));
-  if ((rc = make_chi_octant(c))) return fail(rc);
-  make_third_iterate(c);
+  if ((rc = make_optional(c))) return fail(rc);
   if (tune::enabled() || tune::forced(0) >= 0) {
     if ((rc = tune_level<double>(c))) return fail(rc);
     if (c->opts.precision == 1 && (rc = tune_level<float>(c))) return fail(rc);

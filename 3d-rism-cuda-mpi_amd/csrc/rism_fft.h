@@ -1,5 +1,5 @@
 // rism_fft.h -- LDS-staged mixed-radix (2,3,4,5,6,8,9,10) Stockham FFT of columns,
-// the building block of the axis passes in rism_kernels.hip.
+// the building block of the axis passes in rism_k*pass*.
 //
 // One column (a line of L complex values along one grid axis) is transformed
 // by T threads of a workgroup.  Stage s with radix R performs L/R radix-R

@@ -1,4 +1,4 @@
-// rism_kernels.h -- launch interface of the HIP kernels (rism_kernels.hip).
+// rism_kernels.h -- launch interface of the HIP kernels (rism_k*.hip).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stddef.h>
